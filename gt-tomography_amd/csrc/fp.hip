@@ -60,6 +60,7 @@ struct FPParams {
   double fu, fv, sad, sdd;
   float cx, cy, cz;           // clamp limits in padded texel space (= n_axis + 1)
   unsigned vg;                // column engine: views per launch group (see col_block)
+  unsigned lds_stp;           // column engine: floats of LDS before the parked step lengths
 };
 
 template <typename T>
@@ -283,6 +284,102 @@ __device__ __forceinline__ void wave_lds_sync() {
   __builtin_amdgcn_wave_barrier();
 }
 
+// Voxels z and z + 1 at element e of the z-fastest copy (byte offset of a
+// neighbouring line in soff): one 8-byte load; BF16 takes the four voxels from
+// the even z on and picks two.
+template <typename T>
+__device__ __forceinline__ float2 zpair(__amdgpu_buffer_rsrc_t r, unsigned e, unsigned soff);
+template <>
+__device__ __forceinline__ float2 zpair<float>(__amdgpu_buffer_rsrc_t r, unsigned e, unsigned soff) {
+  return bload2<float>(r, e * 4u, soff);
+}
+template <>
+__device__ __forceinline__ float2 zpair<unsigned short>(__amdgpu_buffer_rsrc_t r, unsigned e,
+                                                        unsigned soff) {
+  const auto v = __builtin_amdgcn_raw_buffer_load_b64(r, (int)((e & ~1u) * 2u), (int)soff, 0);
+  const unsigned w = __builtin_amdgcn_alignbit((unsigned)v[1], (unsigned)v[0], (e & 1u) << 4);
+  return make_float2(__uint_as_float(w << 16), __uint_as_float(w & 0xffff0000u));
+}
+
+// The sum over its n samples of each lane's ray R (lanes with mine unset: 0),
+// for 64 adjacent rows of one detector column whose x/y positions are their
+// own (rays that leave through the volume's top or bottom).  One ray per lane
+// would scatter every load over up to 64 (x, y) lines, since neighbouring rows
+// end at different depths and so step at different lengths; instead a wave
+// takes 8 consecutive samples of 8 adjacent rays at a time and leaves the
+// values in LDS; after the 64 rays' 8 samples each lane adds its own ray's, in
+// order.  Sample positions and the order of the lerps and sums are the per-ray
+// engine's (the same bits).  The texture address unit binds it: it takes four
+// lanes per clock when they hit one line, else one lane per line, so lanes run
+// along a ray (steps of a clipped ray stay within a voxel or two; 28 cache
+// accesses per load) and not across rays (40).  256 x 256 x 160 voxels, 90
+// views of 512 x 384, 30% of the rays clipped: 8.4 ms for the whole
+// projection, 40.8 with one ray per lane.
+//   lds: 64 x 6 floats of ray parameters, 64 x FPG_ROW floats of samples
+constexpr int FPG_ROW = 12;   // 8 samples, 16-byte aligned rows off the same banks
+constexpr int FPG_LDS = 64 * 6 + 64 * FPG_ROW;
+template <typename T>
+__device__ __forceinline__ float fp_gather(const FPParams &P, const RaySetup &R, const bool mine,
+                                           const T *__restrict__ vt, unsigned vt_bytes, int lane,
+                                           float *lds) {
+  const unsigned esz = sizeof(T);
+  const unsigned so_x = P.pz * esz, so_y = P.pzx * esz, so_xy = (P.pzx + P.pz) * esz;
+  const __amdgpu_buffer_rsrc_t rsrc =
+      __builtin_amdgcn_make_buffer_rsrc((void *)vt, (short)0, (int)vt_bytes, 0x00020000);
+  float4 *par4 = reinterpret_cast<float4 *>(lds);
+  float2 *par2 = reinterpret_cast<float2 *>(lds + 64 * 4);
+  float *smp = lds + 64 * 6;
+  par4[lane] = make_float4(R.p[0], R.q[0], R.p[1], R.q[1]);
+  par2[lane] = make_float2(R.p[2], R.q[2]);
+  const unsigned long long rays = __builtin_amdgcn_ballot_w64(mine);
+  wave_lds_sync();
+  const int lr = lane >> 3, ls = lane & 7;
+  float acc = 0.0f;
+  for (int mb = 0; mb < P.n; mb += 8) {
+    const float fm = (float)(mb + ls);
+#pragma unroll 4
+    for (int o = 0; o < 8; ++o) {   // rays 8 o .. 8 o + 7
+      if (!((rays >> (8 * o)) & 0xffull)) continue;
+      const float4 a = par4[8 * o + lr];
+      const float2 b = par2[8 * o + lr];
+      // clamped coordinates are finite and in [0, n + 1]: med3 equals
+      // fminf(fmaxf()), truncation equals floor
+      const float sx = __builtin_amdgcn_fmed3f(fmaf(fm, a.y, a.x), 0.0f, P.cx);
+      const float sy = __builtin_amdgcn_fmed3f(fmaf(fm, a.w, a.z), 0.0f, P.cy);
+      const float sz = __builtin_amdgcn_fmed3f(fmaf(fm, b.y, b.x), 0.0f, P.cz);
+      const float ax = __builtin_amdgcn_fractf(sx), ay = __builtin_amdgcn_fractf(sy);
+      const float az = __builtin_amdgcn_fractf(sz);
+      const unsigned e = ((unsigned)(int)sy * P.px + (unsigned)(int)sx) * P.pz + (unsigned)(int)sz;
+      const float2 v00 = zpair<T>(rsrc, e, 0), v10 = zpair<T>(rsrc, e, so_x);
+      const float2 v01 = zpair<T>(rsrc, e, so_y), v11 = zpair<T>(rsrc, e, so_xy);
+      const float c00 = fmaf(ax, v10.x - v00.x, v00.x);
+      const float c10 = fmaf(ax, v11.x - v01.x, v01.x);
+      const float c01 = fmaf(ax, v10.y - v00.y, v00.y);
+      const float c11 = fmaf(ax, v11.y - v01.y, v01.y);
+      const float c0 = fmaf(ay, c10 - c00, c00);
+      const float c1 = fmaf(ay, c11 - c01, c01);
+      smp[(8 * o + lr) * FPG_ROW + ls] = fmaf(az, c1 - c0, c0);
+    }
+    wave_lds_sync();
+    if (mine) {
+      const int cnt = min(8, P.n - mb);
+      const float4 u = *reinterpret_cast<const float4 *>(&smp[lane * FPG_ROW]);
+      const float4 v = *reinterpret_cast<const float4 *>(&smp[lane * FPG_ROW + 4]);
+      const float x[8] = {u.x, u.y, u.z, u.w, v.x, v.y, v.z, v.w};
+      if (cnt == 8) {
+#pragma unroll
+        for (int t = 0; t < 8; ++t) acc += x[t];
+      } else {
+#pragma unroll
+        for (int t = 0; t < 7; ++t)
+          if (t < cnt) acc += x[t];
+      }
+    }
+    wave_lds_sync();
+  }
+  return acc;
+}
+
 // Block order of the column engine.  xcd_remap gives every XCD a contiguous
 // range of W.  Within it, the blocks of P.vg adjacent views of one (column,
 // row group) come one after another, so they run at the same time on one XCD
@@ -332,71 +429,82 @@ __device__ __forceinline__ void fp_col_body(const FPParams &P, const ViewD *__re
                                             const T *__restrict__ vt, float *__restrict__ proj,
                                             int accumulate, unsigned ngroups, unsigned nblocks,
                                             unsigned vt_bytes) {
-  extern __shared__ float zl[];  // one interpolated z-line (whole 128-wide chunks)
+  extern __shared__ __align__(16) float zl[];  // one interpolated z-line (whole 128-wide chunks)
   int i, grp, k;
   col_block(P, xcd_remap(blockIdx.x, nblocks), ngroups, nblocks, i, grp, k);
   const int lane = threadIdx.x;
-  const ViewD vw = views[k];
-  const ColSetup C = col_setup(P, vw, i);
-  const double a1c = fmax(C.lo, 0.0);
-  const double a2c = fmin(C.hi, 1.0);
-  const bool col_ok = (a2c - a1c) >= 0.0;   // h >= 0 keeps tz monotone in the row
-
   const int row0 = grp * 64 * RPL;
-  float pz[RPL], qz[RPL], acc[RPL], stp[RPL];
+  float pz[RPL], qz[RPL], acc[RPL];
   unsigned shared_mask = 0, valid_mask = 0;
-  int jmin = 0x7fffffff, jmax = -1;
-  RaySetup Rc;  // the column's x/y coordinates (from any shared ray)
-  Rc.p[0] = Rc.p[1] = Rc.q[0] = Rc.q[1] = 0.0f;
+  int gjmin, gjmax;
+  float px0, qx, py0, qy;      // the column's x/y trace
+  float pzl, qzl, pzh, qzh;    // z of the first and last shared rays
+  float *stp = zl + P.lds_stp + lane;   // step lengths, parked in LDS until the end
+  {
+    const ViewD vw = views[k];
+    const ColSetup C = col_setup(P, vw, i);
+    const double a1c = fmax(C.lo, 0.0);
+    const double a2c = fmin(C.hi, 1.0);
+    const bool col_ok = (a2c - a1c) >= 0.0;   // h >= 0 keeps tz monotone in the row
+    // the expressions of ray_finish for the shared (a1, a2), x/y once per column
+    const double span = a2c - a1c, h = span / P.n;
+    px0 = (float)(((C.S0 + a1c * C.d0) / P.lx + 0.5) * P.nx + 0.5);
+    py0 = (float)(((C.S1 + a1c * C.d1) / P.ly + 0.5) * P.ny + 0.5);
+    qx = (float)(C.d0 / P.lx * h * P.nx);
+    qy = (float)(C.d1 / P.ly * h * P.ny);
+    int jmin = 0x7fffffff, jmax = -1;
 #pragma unroll
-  for (int r = 0; r < RPL; ++r) {
-    const int j = row0 + r * 64 + lane;
-    acc[r] = 0.0f;
-    pz[r] = qz[r] = stp[r] = 0.0f;
-    if (j < P.nv) {
-      valid_mask |= 1u << r;
-      const RaySetup R = ray_finish(P, vw, C, j);
-      stp[r] = R.step;
-      pz[r] = R.p[2];
-      qz[r] = R.q[2];
-      if (col_ok && R.a1 == a1c && R.a2 == a2c) {
-        shared_mask |= 1u << r;
-        jmin = min(jmin, j);
-        jmax = max(jmax, j);
-        Rc = R;
+    for (int r = 0; r < RPL; ++r) {
+      const int j = row0 + r * 64 + lane;
+      acc[r] = 0.0f;
+      const double d2 = ((j + 0.5) / P.nv - 0.5) * P.fv + vw.off_v;
+      const double t = fabs(P.lz * 0.5 / d2);   // the z slab is [-t, t]
+      pz[r] = (float)(((a1c * d2) / P.lz + 0.5) * P.nz + 0.5);
+      qz[r] = (float)(d2 / P.lz * h * P.nz);
+      stp[64 * r] = (float)(sqrt(C.d0 * C.d0 + C.d1 * C.d1 + d2 * d2) * fabs(span) / P.n);
+      if (j < P.nv) {
+        valid_mask |= 1u << r;
+        if (col_ok && fmax(fmax(C.lo, -t), 0.0) == a1c && fmin(fmin(C.hi, t), 1.0) == a2c) {
+          shared_mask |= 1u << r;
+          jmin = min(jmin, j);
+          jmax = max(jmax, j);
+        }
       }
+      __builtin_amdgcn_sched_barrier(0);   // one ray's FP64 temporaries at a time
     }
+    gjmin = wave_min_i(jmin);
+    gjmax = wave_max_i(jmax);
   }
-  const int gjmin = wave_min_i(jmin);
-  int gjmax = wave_max_i(jmax);
-
-  RaySetup Rlo, Rhi;
-  if (gjmax >= 0) {
-    // x/y trace and the z range from the first/last shared rays (identical
-    // FP64 code, so identical floats to the per-ray values)
-    Rlo = ray_finish(P, vw, C, gjmin);
-    Rhi = ray_finish(P, vw, C, gjmax);
-    if (SSTEP) {
-      // Every shared ray's z texel coordinate lies between the first and
-      // last shared rays' (monotone in the row) and, being linear in the
-      // step, between its values at the first and last step.  If all four
-      // are inside [0, nz+1] the per-ray z clamp is the identity and is
-      // dropped; otherwise the whole column takes the per-ray path.
-      const float ml = (float)(P.n - 1);
-      const float e0 = Rlo.p[2], e1 = fmaf(ml, Rlo.q[2], Rlo.p[2]);
-      const float e2 = Rhi.p[2], e3 = fmaf(ml, Rhi.q[2], Rhi.p[2]);
-      const bool z_ok = fminf(fminf(e0, e1), fminf(e2, e3)) >= 0.0f &&
-                        fmaxf(fmaxf(e0, e1), fmaxf(e2, e3)) <= P.cz;
-      if (!z_ok) {
-        shared_mask = 0;
-        gjmax = -1;
-      }
+  // from their lanes (0 where there is no shared ray; not used then)
+  auto of_row = [&](const float(&v)[RPL], int j) __attribute__((always_inline)) {
+    const int slot = __builtin_amdgcn_readfirstlane((j - row0) >> 6);
+    float x = 0.0f;
+#pragma unroll
+    for (int r = 0; r < RPL; ++r)
+      if (slot == r) x = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v[r]), (j - row0) & 63));
+    return x;
+  };
+  pzl = of_row(pz, gjmin);
+  qzl = of_row(qz, gjmin);
+  pzh = of_row(pz, gjmax);
+  qzh = of_row(qz, gjmax);
+  if (SSTEP && gjmax >= 0) {
+    // Every shared ray's z texel coordinate lies between the first and last
+    // shared rays' (monotone in the row) and, being linear in the step,
+    // between its values at the first and last step.  If all four are inside
+    // [0, nz+1] the per-ray z clamp is the identity and is dropped; otherwise
+    // the whole column takes the per-ray path.
+    const float ml = (float)(P.n - 1);
+    const float e1 = fmaf(ml, qzl, pzl), e3 = fmaf(ml, qzh, pzh);
+    const bool z_ok = fminf(fminf(pzl, e1), fminf(pzh, e3)) >= 0.0f &&
+                      fmaxf(fmaxf(pzl, e1), fmaxf(pzh, e3)) <= P.cz;
+    if (!z_ok) {
+      shared_mask = 0;
+      gjmax = -1;
     }
   }
 
   if (SSTEP && gjmax >= 0) {
-    const float px0 = Rlo.p[0], qx = Rlo.q[0], py0 = Rlo.p[1], qy = Rlo.q[1];
-    const float pzl = Rlo.p[2], qzl = Rlo.q[2], pzh = Rhi.p[2], qzh = Rhi.q[2];
 #pragma unroll
     for (int r = 0; r < RPL; ++r)
       if (!(shared_mask & (1u << r))) {
@@ -645,8 +753,6 @@ __device__ __forceinline__ void fp_col_body(const FPParams &P, const ViewD *__re
       wave_lds_sync();
     }
   } else if (!SSTEP && gjmax >= 0) {
-    const float px0 = Rlo.p[0], qx = Rlo.q[0], py0 = Rlo.p[1], qy = Rlo.q[1];
-    const float pzl = Rlo.p[2], qzl = Rlo.q[2], pzh = Rhi.p[2], qzh = Rhi.q[2];
     // rays outside the shared set read harmless in-range LDS entries
 #pragma unroll
     for (int r = 0; r < RPL; ++r)
@@ -694,37 +800,27 @@ __device__ __forceinline__ void fp_col_body(const FPParams &P, const ViewD *__re
     }
   }
 
-  // Rays clipped by the z faces (or a column that misses the box): per-ray
-  // loop on the z-fastest layout, same arithmetic order as engine 0.
-  const unsigned todo = valid_mask & ~shared_mask;
-  if (todo) {
+  // the results take the step lengths' places in LDS
 #pragma unroll
+  for (int r = 0; r < RPL; ++r) stp[64 * r] *= acc[r];
+
+  // Rays clipped by the z faces (or a column that misses the box) have x/y
+  // positions of their own: the 64 rows of one register slot together.
+  // The FP64 column setup is evaluated again (through an opaque copy of the
+  // column index), which keeps its 20 registers out of the loops above.
+  const unsigned todo = valid_mask & ~shared_mask;
+  if (__builtin_amdgcn_ballot_w64(todo != 0)) {
+    int iw = __builtin_amdgcn_readfirstlane(i);
+    asm volatile("" : "+s"(iw));
+    const ViewD vw = views[k];
+    const ColSetup C = col_setup(P, vw, iw);
+#pragma nounroll
     for (int r = 0; r < RPL; ++r) {
-      if (!(todo & (1u << r))) continue;
-      const int j = row0 + r * 64 + lane;
-      const RaySetup R = ray_finish(P, vw, C, j);
-      float a = 0.0f;
-      for (int m = 0; m < P.n; ++m) {
-        const float fm = (float)m;
-        const float sx = clampf(fmaf(fm, R.q[0], R.p[0]), P.cx);
-        const float sy = clampf(fmaf(fm, R.q[1], R.p[1]), P.cy);
-        const float sz = clampf(fmaf(fm, R.q[2], R.p[2]), P.cz);
-        const float flx = floorf(sx), fly = floorf(sy), flz = floorf(sz);
-        const float ax = sx - flx, ay = sy - fly, az = sz - flz;
-        const unsigned base = ((unsigned)fly * P.px + (unsigned)flx) * P.pz + (unsigned)flz;
-        const float v000 = ld(vt, base), v100 = ld(vt, base + P.pz);
-        const float v010 = ld(vt, base + P.pzx), v110 = ld(vt, base + P.pzx + P.pz);
-        const float v001 = ld(vt, base + 1), v101 = ld(vt, base + P.pz + 1);
-        const float v011 = ld(vt, base + P.pzx + 1), v111 = ld(vt, base + P.pzx + P.pz + 1);
-        const float c00 = fmaf(ax, v100 - v000, v000);
-        const float c10 = fmaf(ax, v110 - v010, v010);
-        const float c01 = fmaf(ax, v101 - v001, v001);
-        const float c11 = fmaf(ax, v111 - v011, v011);
-        const float c0 = fmaf(ay, c10 - c00, c00);
-        const float c1 = fmaf(ay, c11 - c01, c01);
-        a += fmaf(az, c1 - c0, c0);
-      }
-      acc[r] = a;
+      const bool mine = (todo >> r) & 1u;
+      if (__builtin_amdgcn_ballot_w64(mine) == 0) continue;
+      const RaySetup R = ray_finish(P, vw, C, row0 + r * 64 + lane);
+      const float a = fp_gather<T>(P, R, mine, vt, vt_bytes, lane, zl);
+      if (mine) stp[64 * r] = a * R.step;
     }
   }
 
@@ -733,7 +829,7 @@ __device__ __forceinline__ void fp_col_body(const FPParams &P, const ViewD *__re
     if (!(valid_mask & (1u << r))) continue;
     const int j = row0 + r * 64 + lane;
     const size_t idx = (size_t)i + (size_t)P.nu * ((size_t)j + (size_t)P.nv * k);
-    const float v = acc[r] * stp[r];
+    const float v = stp[64 * r];
     proj[idx] = accumulate ? proj[idx] + v : v;
   }
 }
@@ -890,7 +986,11 @@ void launch_col(const FPParams &P, hipStream_t s, const ViewD *views, const T *v
   const unsigned ngroups = (unsigned)((P.nv + 64 * RPL - 1) / (64 * RPL));
   // one z-line; the cached variants write all NCH chunks of their window
   const size_t zline = ((P.pz + 127) / 128) * 128;
-  const size_t lds = (zline > (size_t)128 * NCH ? zline : (size_t)128 * NCH) * sizeof(float);
+  // and fp_gather's buffers take the same place afterwards
+  const size_t line = std::max({zline, (size_t)128 * NCH, (size_t)FPG_LDS});
+  FPParams Q = P;
+  Q.lds_stp = (unsigned)line;
+  const size_t lds = (line + 64 * RPL) * sizeof(float);
   // a launch covers at most 2^32 - 1 work-items: larger calls go out as
   // several launches over consecutive views (views are independent)
   const size_t per_view = (size_t)P.nu * ngroups;
@@ -901,10 +1001,10 @@ void launch_col(const FPParams &P, hipStream_t s, const ViewD *views, const T *v
     const ViewD *vw = views + v0;
     float *pj = proj + (size_t)v0 * P.nu * P.nv;
     if constexpr (NCH > 0)
-      hipLaunchKernelGGL((k_fp_colc<T, RPL, NCH>), dim3(nblocks), dim3(64), lds, s, P, vw, vt, pj, acc,
+      hipLaunchKernelGGL((k_fp_colc<T, RPL, NCH>), dim3(nblocks), dim3(64), lds, s, Q, vw, vt, pj, acc,
                          ngroups, nblocks, vt_bytes);
     else
-      hipLaunchKernelGGL((k_fp_col<T, RPL, SSTEP, ZP>), dim3(nblocks), dim3(64), lds, s, P, vw, vt, pj,
+      hipLaunchKernelGGL((k_fp_col<T, RPL, SSTEP, ZP>), dim3(nblocks), dim3(64), lds, s, Q, vw, vt, pj,
                          acc, ngroups, nblocks, vt_bytes);
   }
 }
