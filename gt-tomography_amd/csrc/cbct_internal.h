@@ -70,10 +70,11 @@ struct cbct_ctx_s {
   // with the view table
   std::vector<std::pair<std::vector<float>, bool>> bpp_fit_cache;
   int bp_kz = 0;                 // z-voxels per BP thread: 0 = chosen by size, else 8 or 16
-  int fp_max_rpl = 8;            // column engine: most detector rows per lane
+  int fp_max_rpl = 0;            // column engine: most detector rows per lane; 0 = unset (8; engine 1: 12)
   int fp_view_group = 6;         // column engine: adjacent views launched together per column
   int fp_force_variant = 0;      // autotuner trials: variant and tile forced when > 0
   int fp_force_rpl = 0;
+  int fp_force_zc = 0;
   int fp_force_vg = 0;
   int work_dtype = CBCT_F32;     // type of the projectors' working copies of FP32 arrays
   float *d_h = nullptr;          // fp32 spatial kernel, 2*nu entries (h[|m|] mirrored)

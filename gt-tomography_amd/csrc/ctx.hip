@@ -205,6 +205,7 @@ int cbct_ctx_reset(cbct_ctx ctx) {
   ctx->fp_view_group = d.fp_view_group;
   ctx->fp_force_variant = d.fp_force_variant;
   ctx->fp_force_rpl = d.fp_force_rpl;
+  ctx->fp_force_zc = d.fp_force_zc;
   ctx->fp_force_vg = d.fp_force_vg;
   ctx->work_dtype = d.work_dtype;
   ctx->profile = false;

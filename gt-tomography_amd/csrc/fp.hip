@@ -34,6 +34,7 @@
 // Engine 0: one thread per ray, 16x16 detector tiles, x-fastest padded
 // volume, 8 gathers per sample.  Also the basis of the exact transpose.
 #include <algorithm>
+#include <climits>
 #include <cmath>
 #include <map>
 #include <mutex>
@@ -251,28 +252,110 @@ __device__ __forceinline__ float2 bload2<unsigned short>(__amdgpu_buffer_rsrc_t 
   return make_float2(__uint_as_float(w << 16), __uint_as_float(w & 0xffff0000u));
 }
 
-// Two consecutive z as kept in registers by the cached column variant.
-template <typename T>
-struct PairWord;
-template <>
-struct PairWord<float> {
-  using type = unsigned long long;   // both floats in one 64-bit word (kept in registers)
-  __device__ static unsigned long long load(__amdgpu_buffer_rsrc_t r, unsigned voff, unsigned soff) {
-    const auto v = __builtin_amdgcn_raw_buffer_load_b64(r, (int)voff, (int)soff, 0);
-    return (unsigned long long)(unsigned)v[0] | ((unsigned long long)(unsigned)v[1] << 32);
+// a = (a.lo, b.lo), b = (a.hi, b.hi), lo / hi: lanes 0-31 / 32-63
+__device__ __forceinline__ void swap32(unsigned &a, unsigned &b) {
+  const auto r = __builtin_amdgcn_permlane32_swap(a, b, false, false);
+  a = r[0];
+  b = r[1];
+}
+
+// The four corner z-lines (00, 10, 01, 11: x + (line & 1), y + (line >> 1)) of
+// one (x, y) cell over a window of 64 Z z, Z per lane, kept as loaded (BF16
+// pairs stay packed) and unpacked in the combine.  The texture address unit
+// takes four lanes per clock whatever their width, so a load instruction costs
+// it 16 clocks (measured: 8 and 16 bytes per lane the same), and it binds small
+// FP32 windows, whose steps have few vector instructions (80% busy at 128^3).
+//   window piece   FP32                                 BF16
+//   256 z          16 bytes per lane                    (pieces of 128)
+//   192 z          12 bytes per lane                    (128 + 64)
+//   128 z          two lines per load, 16 bytes per     4 bytes per lane
+//                  lane, one in each half of the lanes;
+//                  permlane swaps (fix) then give every
+//                  lane the same z of both
+//   64 z           4 bytes per lane                     2 bytes per lane
+// Two lines per load took 128^3, 180 views, from 0.75 to 0.69 ms; 16 bytes per
+// lane instead of two loads of 8, 512^3, 720 views, from 163 to 156.  BF16
+// steps have the unpacking on top and are bound by the vector unit: wider or
+// shared loads cost them more than they save (512^3, 720 views: 8 or 16 bytes
+// per lane 3% slower; four lines per load at 128^3 0.65 -> 0.72 ms).
+template <typename T, int Z>
+struct Cell {
+  static constexpr bool F = sizeof(T) == 4;
+  static constexpr int Q = F ? Z / 4 : 0, R = Z - 4 * Q;   // 256-z pieces; the rest
+  static constexpr bool TRIPLE = R == 3 && F;
+  static constexpr int PAIRS = TRIPLE ? 0 : R / 2, ONE = R & 1 && !TRIPLE ? 1 : 0;
+  static constexpr int WORDS = F ? Z : PAIRS + ONE;   // per line
+  static constexpr unsigned E = sizeof(T), BP = 256 * E * Q, BO = BP + 128 * E * PAIRS;   // pieces' bytes
+  unsigned w[4][WORDS];
+  unsigned vh;   // lanes' byte offsets when the halves hold different lines
+
+  __device__ __forceinline__ void setup(int lane, unsigned so_x) {
+    vh = 16 * (lane & 31) + (lane & 32 ? so_x : 0);
   }
-  __device__ static float2 unpack(unsigned long long w) {
-    return make_float2(__uint_as_float((unsigned)w), __uint_as_float((unsigned)(w >> 32)));
+  // B: byte offset of line 00 at the window's first z
+  __device__ __forceinline__ void load(__amdgpu_buffer_rsrc_t r, int lane, unsigned B, unsigned so_x,
+                                       unsigned so_y) {
+    const unsigned S[4] = {B, B + so_x, B + so_y, B + so_x + so_y};
+    if constexpr (PAIRS && F) {   // words 2 and 3 of a load are the other line's, after fix
+#pragma unroll
+      for (int c = 0; c < 4; c += 2) {
+        const auto v = __builtin_amdgcn_raw_buffer_load_b128(r, (int)(vh + BP), (int)S[c], 0);
+        w[c][4 * Q] = v[0]; w[c][4 * Q + 1] = v[1]; w[c + 1][4 * Q] = v[2]; w[c + 1][4 * Q + 1] = v[3];
+      }
+    }
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+#pragma unroll
+      for (int q = 0; q < Q; ++q) {
+        const auto v = __builtin_amdgcn_raw_buffer_load_b128(r, (int)(16 * lane + 1024 * q), (int)S[c], 0);
+        w[c][4 * q] = v[0]; w[c][4 * q + 1] = v[1]; w[c][4 * q + 2] = v[2]; w[c][4 * q + 3] = v[3];
+      }
+      if constexpr (TRIPLE) {
+        const auto v = __builtin_amdgcn_raw_buffer_load_b96(r, (int)(12 * lane + BP), (int)S[c], 0);
+        w[c][4 * Q] = v[0]; w[c][4 * Q + 1] = v[1]; w[c][4 * Q + 2] = v[2];
+      }
+      if constexpr (!F) {
+#pragma unroll
+        for (int p = 0; p < PAIRS; ++p)
+          w[c][p] = (unsigned)__builtin_amdgcn_raw_buffer_load_b32(r, (int)(4 * lane + 256 * p), (int)S[c], 0);
+      }
+      if constexpr (ONE) {
+        if constexpr (F) w[c][WORDS - 1] = (unsigned)__builtin_amdgcn_raw_buffer_load_b32(r, (int)(4 * lane + BO), (int)S[c], 0);
+        else w[c][WORDS - 1] = (unsigned)__builtin_amdgcn_raw_buffer_load_b16(r, (int)(2 * lane + BO), (int)S[c], 0);
+      }
+    }
   }
-};
-template <>
-struct PairWord<unsigned short> {
-  using type = unsigned;
-  __device__ static unsigned load(__amdgpu_buffer_rsrc_t r, unsigned voff, unsigned soff) {
-    return (unsigned)__builtin_amdgcn_raw_buffer_load_b32(r, (int)voff, (int)soff, 0);
+  // once per load: the loaded words into their lines' registers
+  __device__ __forceinline__ void fix() {
+    if constexpr (PAIRS && F) {
+#pragma unroll
+      for (int i = 4 * Q; i < 4 * Q + 2; ++i) {
+        swap32(w[0][i], w[1][i]);
+        swap32(w[2][i], w[3][i]);
+      }
+    }
   }
-  __device__ static float2 unpack(unsigned w) {
-    return make_float2(__uint_as_float(w << 16), __uint_as_float(w & 0xffff0000u));
+  // line c's value number t of the lane (in the order of the pieces)
+  __device__ __forceinline__ float at(int c, int t) const {
+    if constexpr (F) return __uint_as_float(w[c][t]);
+    else if (t == Z - 1 && ONE) return __uint_as_float(w[c][WORDS - 1] << 16);
+    else return __uint_as_float(t & 1 ? w[c][t >> 1] & 0xffff0000u : w[c][t >> 1] << 16);
+  }
+  // a lane's Z values to their places of the z-line in LDS
+  static __device__ __forceinline__ void store(float *zl, int lane, const float (&o)[Z]) {
+    int k = 0;
+#pragma unroll
+    for (int q = 0; q < Q; ++q, k += 4)
+      *reinterpret_cast<float4 *>(&zl[256 * q + 4 * lane]) = make_float4(o[k], o[k + 1], o[k + 2], o[k + 3]);
+    if constexpr (TRIPLE) {
+#pragma unroll
+      for (int t = 0; t < 3; ++t) zl[256 * Q + 3 * lane + t] = o[k + t];
+    }
+#pragma unroll
+    for (int p = 0; p < PAIRS; ++p, k += 2)
+      *reinterpret_cast<float2 *>(&zl[256 * Q + 128 * p + (F ? 4 * (lane & 31) + 2 * (lane >> 5) : 2 * lane)]) =
+          make_float2(o[k], o[k + 1]);
+    if constexpr (ONE) zl[256 * Q + 128 * PAIRS + lane] = o[k];
   }
 };
 
@@ -411,20 +494,14 @@ __device__ __forceinline__ void col_block(const FPParams &P, unsigned W, unsigne
 //     z clamp (a column-level range check instead), two consecutive z per
 //     lane and load (BF16 storage: one dword per lane instead of two 16-bit
 //     loads, 1.5x faster there).
-//   NCH > 0 (with SSTEP, ZP = 2): the z window of the whole ray (all its
-//     steps, all shared rows) is fixed once; when it spans at most NCH
-//     chunks of 128 z, the four corner z-lines of the current (x, y) cell
-//     stay in registers while the ray stays in the cell.  FP32 copies: a
-//     step into a neighbouring cell keeps the lines the two cells share (two
-//     of four for a move along x or y, one for a diagonal move) and loads
-//     only the others; the column's (x, y) is wave-uniform, so the case
-//     split is a scalar branch, and the lines are kept as (00, 10, 01, 11)
-//     of the cell and shifted by register moves.  BF16 copies: all four are
-//     reloaded for the next step's cell right after this step's combine.
-//     Every line load fetches all NCH chunks (no per-chunk branches); chunks
-//     past the window are never read.
+//   ZC > 0 (with SSTEP, ZP = 2): the z window of the whole ray (all its steps,
+//     all shared rows) is fixed once; when it spans at most 64 ZC z, the four
+//     corner z-lines of the current (x, y) cell stay in registers while the
+//     ray stays in the cell (Cell) and all four are reloaded for the next
+//     step's cell right after this step's combine.  Every load fetches the
+//     whole window; z past the part a step needs are never read.
 // All produce the same bits as the per-ray engine.
-template <typename T, int RPL, bool SSTEP, int ZP, int NCH>
+template <typename T, int RPL, bool SSTEP, int ZP, int ZC>
 __device__ __forceinline__ void fp_col_body(const FPParams &P, const ViewD *__restrict__ views,
                                             const T *__restrict__ vt, float *__restrict__ proj,
                                             int accumulate, unsigned ngroups, unsigned nblocks,
@@ -518,100 +595,37 @@ __device__ __forceinline__ void fp_col_body(const FPParams &P, const ViewD *__re
         __builtin_amdgcn_make_buffer_rsrc((void *)vt, (short)0, (int)vt_bytes, 0x00020000);
     const unsigned lane_off = (unsigned)lane * esz;
     bool done = false;
-    if constexpr (NCH > 0) {
-      static_assert(ZP == 2, "cached z-lines use pair loads");
+    if constexpr (ZC > 0) {
       // The window: per step the rays read z in [zlo(m), zhi(m)], both linear
       // in m through the same fmaf as below (so monotone), hence extreme at
       // the first or last step.
       const float ml = (float)(P.n - 1);
       const int zlo_min = __builtin_amdgcn_readfirstlane((int)fminf(pzl, fmaf(ml, qzl, pzl)));
       const int zhi_max = __builtin_amdgcn_readfirstlane((int)fmaxf(pzh, fmaf(ml, qzh, pzh))) + 1;
-      const int zb0 = zlo_min & ~1;
-      const int nchw = (zhi_max - zb0 + 128) >> 7;
+      const int zb0 = zlo_min & ~3;   // pieces aligned to their width
       // (cell coordinates are packed as two 16-bit halves below)
-      if (nchw <= NCH && P.cx < 65535.0f && P.cy < 65535.0f) {
+      if (zhi_max - zb0 < 64 * ZC && P.cx < 65535.0f && P.cy < 65535.0f) {
         done = true;
-        // the lines as loaded: FP32 pairs, or BF16 pairs packed in one word
-        // (unpacked in the combine, which keeps the registers, and with them
-        // the occupancy, of the uncached variant)
-        using PW = PairWord<T>;
-        using W = typename PW::type;
-        W L00[NCH], L10[NCH], L01[NCH], L11[NCH];
+        Cell<T, ZC> L;
+        L.setup(lane, so_x);
         const unsigned zoff = (unsigned)zb0 * esz;
-        int cx = -8, cy = -8;   // no cell loaded yet
-        auto load_line = [&](W(&L)[NCH], unsigned B) __attribute__((always_inline)) {
-#pragma unroll
-          for (int c = 0; c < NCH; ++c) L[c] = PW::load(rsrc, 2 * lane_off + (unsigned)(128 * c) * esz, B);
-        };
-        auto copy_line = [&](W(&D)[NCH], const W(&S)[NCH]) __attribute__((always_inline)) {
-#pragma unroll
-          for (int c = 0; c < NCH; ++c) D[c] = S[c];
-        };
         const float *zb = zl - zb0;
         // all four lines of cell (ix, iy)
         auto load_cell = [&](int ix, int iy) __attribute__((always_inline)) {
-          const unsigned B = ((unsigned)iy * P.px + (unsigned)ix) * PZ * esz + zoff;
-          load_line(L00, B); load_line(L10, B + so_x);
-          load_line(L01, B + so_y); load_line(L11, B + so_xy);
-        };
-        // the four lines of cell (ix, iy), keeping those shared with the
-        // current cell (FP32 copies, bound by their line bytes)
-        auto update_cell = [&](int ix, int iy) __attribute__((always_inline)) {
-            if (ix != cx || iy != cy) {
-              const int dx = ix - cx, dy = iy - cy;
-              const unsigned B = ((unsigned)iy * P.px + (unsigned)ix) * PZ * esz + zoff;
-              if (dy == 0 && dx == 1) {
-                copy_line(L00, L10); copy_line(L01, L11);
-                load_line(L10, B + so_x); load_line(L11, B + so_xy);
-              } else if (dy == 0 && dx == -1) {
-                copy_line(L10, L00); copy_line(L11, L01);
-                load_line(L00, B); load_line(L01, B + so_y);
-              } else if (dx == 0 && dy == 1) {
-                copy_line(L00, L01); copy_line(L10, L11);
-                load_line(L01, B + so_y); load_line(L11, B + so_xy);
-              } else if (dx == 0 && dy == -1) {
-                copy_line(L01, L00); copy_line(L11, L10);
-                load_line(L00, B); load_line(L10, B + so_x);
-              } else if (dx == 1 && dy == 1) {
-                copy_line(L00, L11);
-                load_line(L10, B + so_x); load_line(L01, B + so_y); load_line(L11, B + so_xy);
-              } else if (dx == 1 && dy == -1) {
-                copy_line(L01, L10);
-                load_line(L00, B); load_line(L10, B + so_x); load_line(L11, B + so_xy);
-              } else if (dx == -1 && dy == 1) {
-                copy_line(L10, L01);
-                load_line(L00, B); load_line(L01, B + so_y); load_line(L11, B + so_xy);
-              } else if (dx == -1 && dy == -1) {
-                copy_line(L11, L00);
-                load_line(L00, B); load_line(L10, B + so_x); load_line(L01, B + so_y);
-              } else {
-                load_line(L00, B); load_line(L10, B + so_x);
-                load_line(L01, B + so_y); load_line(L11, B + so_xy);
-              }
-              cx = ix;
-              cy = iy;
-            }
+          L.load(rsrc, lane, ((unsigned)iy * P.px + (unsigned)ix) * PZ * esz + zoff, so_x, so_y);
         };
         // the combined z-line of the cell's lines into LDS
         auto combine = [&](const float ax, const float ay) __attribute__((always_inline)) {
+          float o[ZC];
 #pragma unroll
-            for (int c = 0; c < NCH; ++c) {
-              const float2 v00 = PairWord<T>::unpack(L00[c]), v10 = PairWord<T>::unpack(L10[c]);
-              const float2 v01 = PairWord<T>::unpack(L01[c]), v11 = PairWord<T>::unpack(L11[c]);
-              float2 o;
-              {
-                const float c0 = fmaf(ax, v10.x - v00.x, v00.x);
-                const float c1 = fmaf(ax, v11.x - v01.x, v01.x);
-                o.x = fmaf(ay, c1 - c0, c0);
-              }
-              {
-                const float c0 = fmaf(ax, v10.y - v00.y, v00.y);
-                const float c1 = fmaf(ax, v11.y - v01.y, v01.y);
-                o.y = fmaf(ay, c1 - c0, c0);
-              }
-              *reinterpret_cast<float2 *>(&zl[2 * lane + 128 * c]) = o;
-            }
-            wave_lds_sync();
+          for (int t = 0; t < ZC; ++t) {
+            const float v00 = L.at(0, t), v01 = L.at(2, t);
+            const float c0 = fmaf(ax, L.at(1, t) - v00, v00);
+            const float c1 = fmaf(ax, L.at(3, t) - v01, v01);
+            o[t] = fmaf(ay, c1 - c0, c0);
+          }
+          L.store(zl, lane, o);
+          wave_lds_sync();
         };
         // every ray's z-lerp from the combined z-line
         auto rays = [&](const float fm) __attribute__((always_inline)) {
@@ -625,66 +639,47 @@ __device__ __forceinline__ void fp_col_body(const FPParams &P, const ViewD *__re
             }
             wave_lds_sync();
         };
-        // one step with FP32 copies
-        auto step = [&](const float fm, const float ax, const float ay, const int ix,
-                        const int iy) __attribute__((always_inline)) {
-          update_cell(ix, iy);
-          combine(ax, ay);
-          rays(fm);
-        };
-        // BF16 copies: the x/y part of a step, the same for the whole wave,
-        // is evaluated for 64 steps at once, step mb + lane in each lane (the
-        // same expressions as per step, so the same values), and each step
-        // reads its cell and weights back into scalar registers.  The lines
-        // of the next step's cell, when it changes, are all four reloaded
-        // straight into their registers once this step's combine has used
-        // them, so they arrive while this step's rays run (fewer
-        // instructions than keeping the shared lines, whose register moves
-        // wait on the new loads).  FP32 copies: per-step setup and shared
-        // lines kept (measured faster there).
-        if constexpr (sizeof(T) == 2) {
-          {
-            const float sx = __builtin_amdgcn_fmed3f(fmaf(0.0f, qx, px0), 0.0f, P.cx);
-            const float sy = __builtin_amdgcn_fmed3f(fmaf(0.0f, qy, py0), 0.0f, P.cy);
-            cx = __builtin_amdgcn_readfirstlane((int)sx);
-            cy = __builtin_amdgcn_readfirstlane((int)sy);
-            load_cell(cx, cy);
-          }
-          for (int mb = 0; mb < P.n; mb += 64) {
-            const float fml = (float)(mb + lane);
-            const float sxl = __builtin_amdgcn_fmed3f(fmaf(fml, qx, px0), 0.0f, P.cx);
-            const float syl = __builtin_amdgcn_fmed3f(fmaf(fml, qy, py0), 0.0f, P.cy);
-            const int axl = __float_as_int(__builtin_amdgcn_fractf(sxl));
-            const int ayl = __float_as_int(__builtin_amdgcn_fractf(syl));
-            // cell of step mb + lane + 1 (the next step's)
-            const float fmn = (float)(mb + lane + 1);
-            const float sxn = __builtin_amdgcn_fmed3f(fmaf(fmn, qx, px0), 0.0f, P.cx);
-            const float syn = __builtin_amdgcn_fmed3f(fmaf(fmn, qy, py0), 0.0f, P.cy);
-            const int cn = (int)((unsigned)sxn | ((unsigned)syn << 16));
-            const int cnt = __builtin_amdgcn_readfirstlane(min(64, P.n - mb));
-            for (int l = 0; l < cnt; ++l) {
-              const float ax = __int_as_float(__builtin_amdgcn_readlane(axl, l));
-              const float ay = __int_as_float(__builtin_amdgcn_readlane(ayl, l));
-              combine(ax, ay);
-              const unsigned c = (unsigned)__builtin_amdgcn_readlane(cn, l);
-              const int nx = (int)(c & 0xffffu), ny = (int)(c >> 16);
-              if (mb + l + 1 < P.n && (nx != cx || ny != cy)) {
-                load_cell(nx, ny);
-                cx = nx;
-                cy = ny;
-              }
-              rays((float)(mb + l));
+        // The x/y part of a step, the same for the whole wave, is evaluated for
+        // 64 steps at once, step mb + lane in each lane (the same expressions
+        // as per step, so the same values), and each step reads its cell and
+        // weights back into scalar registers.  The lines of the next step's
+        // cell, when it changes, are all four reloaded straight into their
+        // registers once this step's combine has used them, so they arrive
+        // while this step's rays run.  Keeping the lines that the two cells
+        // share saves half the bytes, but the register moves wait on the loads:
+        // 13.1 against 12.6 ms (FP32 copies, 512^3, 48 views).
+        const float s0x = __builtin_amdgcn_fmed3f(fmaf(0.0f, qx, px0), 0.0f, P.cx);
+        const float s0y = __builtin_amdgcn_fmed3f(fmaf(0.0f, qy, py0), 0.0f, P.cy);
+        int cx = __builtin_amdgcn_readfirstlane((int)s0x), cy = __builtin_amdgcn_readfirstlane((int)s0y);
+        load_cell(cx, cy);
+        bool fresh = true;   // loaded and not yet fixed
+        for (int mb = 0; mb < P.n; mb += 64) {
+          const float fml = (float)(mb + lane);
+          const float sxl = __builtin_amdgcn_fmed3f(fmaf(fml, qx, px0), 0.0f, P.cx);
+          const float syl = __builtin_amdgcn_fmed3f(fmaf(fml, qy, py0), 0.0f, P.cy);
+          const int axl = __float_as_int(__builtin_amdgcn_fractf(sxl));
+          const int ayl = __float_as_int(__builtin_amdgcn_fractf(syl));
+          // cell of step mb + lane + 1 (the next step's)
+          const float fmn = (float)(mb + lane + 1);
+          const float sxn = __builtin_amdgcn_fmed3f(fmaf(fmn, qx, px0), 0.0f, P.cx);
+          const float syn = __builtin_amdgcn_fmed3f(fmaf(fmn, qy, py0), 0.0f, P.cy);
+          const int cn = (int)((unsigned)sxn | ((unsigned)syn << 16));
+          const int cnt = __builtin_amdgcn_readfirstlane(min(64, P.n - mb));
+          for (int l = 0; l < cnt; ++l) {
+            const float ax = __int_as_float(__builtin_amdgcn_readlane(axl, l));
+            const float ay = __int_as_float(__builtin_amdgcn_readlane(ayl, l));
+            if (fresh) L.fix();
+            combine(ax, ay);
+            const unsigned c = (unsigned)__builtin_amdgcn_readlane(cn, l);
+            const int nx = (int)(c & 0xffffu), ny = (int)(c >> 16);
+            fresh = mb + l + 1 < P.n && (nx != cx || ny != cy);
+            if (fresh) {
+              load_cell(nx, ny);
+              cx = nx;
+              cy = ny;
             }
+            rays((float)(mb + l));
           }
-        }
-        for (int m = 0; sizeof(T) != 2 && m < P.n; ++m) {
-          const float fm = (float)m;
-          const float sx = __builtin_amdgcn_fmed3f(fmaf(fm, qx, px0), 0.0f, P.cx);
-          const float sy = __builtin_amdgcn_fmed3f(fmaf(fm, qy, py0), 0.0f, P.cy);
-          const float ax = __builtin_amdgcn_fractf(sx), ay = __builtin_amdgcn_fractf(sy);
-          const int ix = __builtin_amdgcn_readfirstlane((int)sx);
-          const int iy = __builtin_amdgcn_readfirstlane((int)sy);
-          step(fm, ax, ay, ix, iy);
         }
       }
     }
@@ -842,17 +837,18 @@ __global__ void __launch_bounds__(64) k_fp_col(FPParams P, const ViewD *__restri
   fp_col_body<T, RPL, SSTEP, ZP, 0>(P, views, vt, proj, accumulate, ngroups, nblocks, vt_bytes);
 }
 
-// The cached variant, held to five waves per SIMD (five measured faster than
-// four with more registers, and than six with BF16 copies).  With FP32
-// copies and 6 rows per lane, five waves spill 3 VGPRs to scratch; four
-// waves without the spill measured slower (162 against 143 ms at 512^3 x
-// 720 views).
-template <typename T, int RPL, int NCH>
-__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(5)))
+// The cached variant, held to five waves per SIMD, four from 8 rows per lane on
+// (more rows spill at five).  512^3, 48 views, 6 rows per lane: four / five /
+// six / seven waves 12.8 / 12.8 / 14.1 / 15.2 ms (FP32 copies), 11.0 / 11.1 /
+// 11.2 / 12.3 (BF16); 291^3, 32 views, 8 rows: 1.61 / 1.70 / 2.03 / 2.19 and
+// 1.49 / 1.57 / 1.63 / 1.82.
+constexpr int colc_waves(int rpl) { return rpl >= 8 ? 4 : 5; }
+template <typename T, int RPL, int ZC>
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(colc_waves(RPL))))
 k_fp_colc(FPParams P, const ViewD *__restrict__ views, const T *__restrict__ vt,
           float *__restrict__ proj, int accumulate, unsigned ngroups, unsigned nblocks,
           unsigned vt_bytes) {
-  fp_col_body<T, RPL, true, 2, NCH>(P, views, vt, proj, accumulate, ngroups, nblocks, vt_bytes);
+  fp_col_body<T, RPL, true, 2, ZC>(P, views, vt, proj, accumulate, ngroups, nblocks, vt_bytes);
 }
 
 // ------------------------------------------------------------ layouts
@@ -980,14 +976,14 @@ int make_params(cbct_ctx ctx, const cbct_geom *g, float spp, FPParams &P) {
   return CBCT_OK;
 }
 
-template <typename T, int RPL, bool SSTEP, int ZP, int NCH>
+template <typename T, int RPL, bool SSTEP, int ZP, int ZC>
 void launch_col(const FPParams &P, hipStream_t s, const ViewD *views, const T *vt, float *proj,
                 int acc, int nviews, unsigned vt_bytes) {
   const unsigned ngroups = (unsigned)((P.nv + 64 * RPL - 1) / (64 * RPL));
-  // one z-line; the cached variants write all NCH chunks of their window
+  // one z-line; the cached variants write their whole window
   const size_t zline = ((P.pz + 127) / 128) * 128;
   // and fp_gather's buffers take the same place afterwards
-  const size_t line = std::max({zline, (size_t)128 * NCH, (size_t)FPG_LDS});
+  const size_t line = std::max({zline, (size_t)64 * ZC, (size_t)FPG_LDS});
   FPParams Q = P;
   Q.lds_stp = (unsigned)line;
   const size_t lds = (line + 64 * RPL) * sizeof(float);
@@ -1000,8 +996,8 @@ void launch_col(const FPParams &P, hipStream_t s, const ViewD *views, const T *v
     const unsigned nblocks = (unsigned)(per_view * (size_t)nvc);
     const ViewD *vw = views + v0;
     float *pj = proj + (size_t)v0 * P.nu * P.nv;
-    if constexpr (NCH > 0)
-      hipLaunchKernelGGL((k_fp_colc<T, RPL, NCH>), dim3(nblocks), dim3(64), lds, s, Q, vw, vt, pj, acc,
+    if constexpr (ZC > 0)
+      hipLaunchKernelGGL((k_fp_colc<T, RPL, ZC>), dim3(nblocks), dim3(64), lds, s, Q, vw, vt, pj, acc,
                          ngroups, nblocks, vt_bytes);
     else
       hipLaunchKernelGGL((k_fp_col<T, RPL, SSTEP, ZP>), dim3(nblocks), dim3(64), lds, s, Q, vw, vt, pj,
@@ -1009,20 +1005,36 @@ void launch_col(const FPParams &P, hipStream_t s, const ViewD *views, const T *v
   }
 }
 
-// variant 1: vector step setup, one z per load; variant 2: scalar step
-// setup, two z per load; variants 3 and 4: variant 2 with the corner z-lines
-// cached in registers over a whole-ray window of at most 2 (3: 3) chunks of
-// 128 z (k_fp_colc).
+// Column-engine variant and tile.  variant 0: per ray; 1: vector step setup,
+// one z per load; 2: scalar step setup, two z per load; 3: variant 2 with the
+// corner z-lines cached in registers over a whole-ray window of at most 64 zc z
+// (k_fp_colc), zc z per lane.
+struct FPChoice {
+  int variant;
+  int rpl;      // rows per lane
+  int zc = 0;
+  int vg = 0;   // views per launch group; 0 = the context's setting
+};
+
 template <typename T, int RPL>
-void launch_col_w(const FPParams &P, int variant, hipStream_t s, const ViewD *views, const T *vt,
+void launch_col_w(const FPParams &P, const FPChoice &c, hipStream_t s, const ViewD *views, const T *vt,
                   float *proj, int acc, int nviews, unsigned vt_bytes) {
-  switch (variant) {
-    case 2: launch_col<T, RPL, true, 2, 0>(P, s, views, vt, proj, acc, nviews, vt_bytes); break;
-    case 3: launch_col<T, RPL, true, 2, 2>(P, s, views, vt, proj, acc, nviews, vt_bytes); break;
-    case 4: launch_col<T, RPL, true, 2, 3>(P, s, views, vt, proj, acc, nviews, vt_bytes); break;
-    default: launch_col<T, RPL, false, 1, 0>(P, s, views, vt, proj, acc, nviews, vt_bytes); break;
+  if (c.variant == 1) return launch_col<T, RPL, false, 1, 0>(P, s, views, vt, proj, acc, nviews, vt_bytes);
+  if (c.variant == 2) return launch_col<T, RPL, true, 2, 0>(P, s, views, vt, proj, acc, nviews, vt_bytes);
+  switch (c.zc) {
+    case 1: launch_col<T, RPL, true, 2, 1>(P, s, views, vt, proj, acc, nviews, vt_bytes); break;
+    case 2: launch_col<T, RPL, true, 2, 2>(P, s, views, vt, proj, acc, nviews, vt_bytes); break;
+    case 3: launch_col<T, RPL, true, 2, 3>(P, s, views, vt, proj, acc, nviews, vt_bytes); break;
+    case 4: launch_col<T, RPL, true, 2, 4>(P, s, views, vt, proj, acc, nviews, vt_bytes); break;
+    case 5: launch_col<T, RPL, true, 2, 5>(P, s, views, vt, proj, acc, nviews, vt_bytes); break;
+    default: launch_col<T, RPL, true, 2, 6>(P, s, views, vt, proj, acc, nviews, vt_bytes); break;
   }
 }
+
+// Most rows per lane and most z per lane of a cached line.
+constexpr int FP_RPL_MAX = 12, FP_ZC_MAX = 6;
+// Configured tile; unset: 8 (engine 1 chooses by itself, see default_variant).
+inline int col_tile(const cbct_ctx ctx) { return ctx->fp_max_rpl ? ctx->fp_max_rpl : 8; }
 
 // Rows per lane that dispatch_col picks for max_rpl.
 inline int rows_per_lane(int nv, int max_rpl) {
@@ -1035,69 +1047,85 @@ inline int rows_per_lane(int nv, int max_rpl) {
 // into equal groups of whole 64-row blocks).  More rows per wave share one
 // z-line load; fewer keep registers, and so occupancy, in check.
 template <typename T>
-void dispatch_col(const FPParams &P, int variant, int rpl, hipStream_t s, const ViewD *views,
-                  const T *vt, float *proj, int acc, int nviews, unsigned vt_bytes) {
-  switch (rpl) {
-    case 1: launch_col_w<T, 1>(P, variant, s, views, vt, proj, acc, nviews, vt_bytes); break;
-    case 2: launch_col_w<T, 2>(P, variant, s, views, vt, proj, acc, nviews, vt_bytes); break;
-    case 3: launch_col_w<T, 3>(P, variant, s, views, vt, proj, acc, nviews, vt_bytes); break;
-    case 4: launch_col_w<T, 4>(P, variant, s, views, vt, proj, acc, nviews, vt_bytes); break;
-    case 5: launch_col_w<T, 5>(P, variant, s, views, vt, proj, acc, nviews, vt_bytes); break;
-    case 6: launch_col_w<T, 6>(P, variant, s, views, vt, proj, acc, nviews, vt_bytes); break;
-    case 7: launch_col_w<T, 7>(P, variant, s, views, vt, proj, acc, nviews, vt_bytes); break;
-    case 8: launch_col_w<T, 8>(P, variant, s, views, vt, proj, acc, nviews, vt_bytes); break;
-    case 9: launch_col_w<T, 9>(P, variant, s, views, vt, proj, acc, nviews, vt_bytes); break;
-    case 10: launch_col_w<T, 10>(P, variant, s, views, vt, proj, acc, nviews, vt_bytes); break;
-    case 11: launch_col_w<T, 11>(P, variant, s, views, vt, proj, acc, nviews, vt_bytes); break;
-    default: launch_col_w<T, 12>(P, variant, s, views, vt, proj, acc, nviews, vt_bytes); break;
+void dispatch_col(const FPParams &P, const FPChoice &c, hipStream_t s, const ViewD *views, const T *vt,
+                  float *proj, int acc, int nviews, unsigned vt_bytes) {
+  switch (c.rpl) {
+    case 1: launch_col_w<T, 1>(P, c, s, views, vt, proj, acc, nviews, vt_bytes); break;
+    case 2: launch_col_w<T, 2>(P, c, s, views, vt, proj, acc, nviews, vt_bytes); break;
+    case 3: launch_col_w<T, 3>(P, c, s, views, vt, proj, acc, nviews, vt_bytes); break;
+    case 4: launch_col_w<T, 4>(P, c, s, views, vt, proj, acc, nviews, vt_bytes); break;
+    case 5: launch_col_w<T, 5>(P, c, s, views, vt, proj, acc, nviews, vt_bytes); break;
+    case 6: launch_col_w<T, 6>(P, c, s, views, vt, proj, acc, nviews, vt_bytes); break;
+    case 7: launch_col_w<T, 7>(P, c, s, views, vt, proj, acc, nviews, vt_bytes); break;
+    case 8: launch_col_w<T, 8>(P, c, s, views, vt, proj, acc, nviews, vt_bytes); break;
+    case 9: launch_col_w<T, 9>(P, c, s, views, vt, proj, acc, nviews, vt_bytes); break;
+    case 10: launch_col_w<T, 10>(P, c, s, views, vt, proj, acc, nviews, vt_bytes); break;
+    case 11: launch_col_w<T, 11>(P, c, s, views, vt, proj, acc, nviews, vt_bytes); break;
+    default: launch_col_w<T, 12>(P, c, s, views, vt, proj, acc, nviews, vt_bytes); break;
   }
 }
 
-// Engine 1's choice.  The cached variant pays when every row group's
-// whole-ray z window fits its two chunks.  A bound: a ray through detector
-// height v (offset included) is at z = v t / SDD where t, its depth along the
-// central ray, lies in [SAD - R, SAD + R] inside the box (R: half the box's
-// xy diagonal); the window spans the extremes of v t over the group's rows
-// and that depth range, plus the texel, the alignment and rounding slack.
-// The largest tile (rows per lane, at least 2) whose groups fit is taken;
-// if none does, the per-step variant measured fastest for the storage type
-// with the configured tile.
-struct FPChoice {
-  int variant;
-  int rpl;
-  int vg = 0;   // views per launch group; 0 = the context's setting
-};
-
+// Bound on a row group's whole-ray z window in voxels, over all groups of rpl
+// rows per lane.  A ray through detector height v (offset included) is at z =
+// v t / SDD where t, its depth along the central ray, lies in [SAD - R, SAD + R]
+// inside the box (R: half the box's xy diagonal); the window spans the extremes
+// of v t over the group's rows and that depth range, no further than the box
+// itself (rays that leave through its top or bottom are not shared), plus the
+// texel, the window's alignment (3) and rounding slack.
 double window_bound(const cbct_geom *g, int nv, int rpl, float omin, float omax) {
   const double R = 0.5 * std::sqrt((double)g->lx * g->lx + (double)g->ly * g->ly);
   const double t0 = (double)g->sad - R, t1 = (double)g->sad + R;
-  const double pitch = (double)g->fov_v / nv, vz = (double)g->lz / g->nz;
+  const double pitch = (double)g->fov_v / nv, vz = (double)g->lz / g->nz, hz = 0.5 * g->lz;
   double worst = 0.0;
   for (int row0 = 0; row0 < nv; row0 += 64 * rpl) {
     const int row1 = std::min(nv, row0 + 64 * rpl) - 1;
     const double v0 = ((row0 + 0.5) / nv - 0.5) * g->fov_v + omin - 0.5 * pitch;
     const double v1 = ((row1 + 0.5) / nv - 0.5) * g->fov_v + omax + 0.5 * pitch;
     const double e[4] = {v0 * t0, v0 * t1, v1 * t0, v1 * t1};
-    const double lo = std::min(std::min(e[0], e[1]), std::min(e[2], e[3]));
-    const double hi = std::max(std::max(e[0], e[1]), std::max(e[2], e[3]));
-    worst = std::max(worst, (hi - lo) / g->sdd / vz);
+    const double lo = std::min(std::min(e[0], e[1]), std::min(e[2], e[3])) / g->sdd;
+    const double hi = std::max(std::max(e[0], e[1]), std::max(e[2], e[3])) / g->sdd;
+    worst = std::max(worst, (std::min(hi, hz) - std::max(lo, -hz)) / vz);
   }
-  return worst + 4.0;
+  return worst + 6.0;
 }
 
-FPChoice default_variant(cbct_ctx ctx, const cbct_geom *g, const FPParams &P, int view0, int nviews,
-                         int per_step) {
+// z per lane of the cached variant whose window holds every row group at rpl
+// rows per lane (may exceed FP_ZC_MAX: no such variant).
+int window_zc(cbct_ctx ctx, const cbct_geom *g, int nv, int rpl, int view0, int nviews) {
   float omin = 0.0f, omax = 0.0f;
   for (int k = 0; k < nviews; ++k) {
     const float ov = ctx->offsets[2 * (size_t)(view0 + k) + 1];
     omin = k ? fminf(omin, ov) : ov;
     omax = k ? fmaxf(omax, ov) : ov;
   }
-  for (int r = ctx->fp_max_rpl; r >= 2; --r) {
+  return (int)std::min(1e6, std::ceil(window_bound(g, nv, rpl, omin, omax) / 64.0));
+}
+
+// Engine 1's choice: the cached variant with the tile (rows per lane) and the
+// window (64 zc z) that cost least per step over the whole column, among those
+// whose window fits.  A step of one wave costs about 12 vector instructions, 7
+// per row and lane and, per z and lane, 6 (FP32 copies) or 10 (BF16, unpacking
+// included); a column has as many waves as row groups.  Measured beside it
+// (FP32 copies): 128^3, 180 views, 192 rows: rpl 3 with zc 2 0.69 ms, zc 3 0.80,
+// zc 4 0.97; rpl 2 in two groups 1.21; 291^3, 32 views, 500 rows: rpl 8 with zc 5
+// 1.56 ms, 4 with 3 1.98, 3 with 2 2.15; 512^3, 48 views, 768 rows: 6 with 4
+// 12.6, 4 with 3 13.9, 3 with 3 17.2.  Windows wider than 384 z take the
+// per-step variant measured fastest for the storage type.
+FPChoice default_variant(cbct_ctx ctx, const cbct_geom *g, const FPParams &P, int view0, int nviews,
+                         size_t esz, int per_step) {
+  FPChoice best{per_step, rows_per_lane(P.nv, col_tile(ctx))};
+  int best_cost = INT_MAX;
+  for (int r = ctx->fp_max_rpl ? ctx->fp_max_rpl : FP_RPL_MAX; r >= 1; --r) {
     const int rpl = rows_per_lane(P.nv, r);
-    if (rpl >= 2 && window_bound(g, P.nv, rpl, omin, omax) <= 256.0) return {3, rpl};
+    const int zc = window_zc(ctx, g, P.nv, rpl, view0, nviews);
+    const int groups = (P.nv + 64 * rpl - 1) / (64 * rpl);
+    const int cost = groups * (12 + 7 * rpl + (esz == 2 ? 10 : 6) * zc);
+    if (zc <= FP_ZC_MAX && cost < best_cost) {
+      best_cost = cost;
+      best = {3, rpl, zc};
+    }
   }
-  return {per_step, rows_per_lane(P.nv, ctx->fp_max_rpl)};
+  return best;
 }
 
 // Autotuned choices, process-wide (cbct_fp_autotune): the geometry, the
@@ -1131,19 +1159,20 @@ FPChoice select_variant(cbct_ctx ctx, const cbct_geom *g, const FPParams &P, int
                         size_t esz, float spp) {
   const size_t vt_bytes = (size_t)P.pzx * padded_dim(g->ny) * esz;
   const size_t zline_bytes = ((P.pz + 127) / 128) * 128 * sizeof(float);
-  const int rpl = rows_per_lane(P.nv, ctx->fp_max_rpl);
+  const int rpl = rows_per_lane(P.nv, col_tile(ctx));
   if (ctx->fp_engine == 0 || vt_bytes + (size_t)P.pzx * esz * 2 >= (1ull << 31) || zline_bytes > 65536)
     return {0, rpl};
-  if (ctx->fp_force_variant > 0) return {ctx->fp_force_variant, ctx->fp_force_rpl, ctx->fp_force_vg};
+  if (ctx->fp_force_variant > 0)
+    return {ctx->fp_force_variant, ctx->fp_force_rpl, ctx->fp_force_zc, ctx->fp_force_vg};
   const int per_step = esz == 2 ? 2 : 1;
   if (ctx->fp_engine == 2) return {3 - per_step, rpl};
-  if (ctx->fp_engine >= 3) return {ctx->fp_engine, rpl};
+  if (ctx->fp_engine >= 3) return {3, rpl, ctx->fp_engine == 3 ? 4 : 6};
   {
     std::lock_guard<std::mutex> lk(g_tune_mu);
     auto it = g_tuned.find(tune_key(g, spp, esz));
     if (it != g_tuned.end()) return it->second.choice;
   }
-  return default_variant(ctx, g, P, view0, nviews, per_step);
+  return default_variant(ctx, g, P, view0, nviews, esz, per_step);
 }
 
 // Bytes of the padded working copy cbct_fp builds for this call (the
@@ -1200,8 +1229,7 @@ int run_fp(cbct_ctx ctx, const cbct_geom *g, const FPParams &P, int view0, int n
   FPParams Q = P;
   if (choice.vg > 0) Q.vg = (unsigned)choice.vg;
   cbct_prof_mark(ctx, PROF_FP, 0, s);
-  dispatch_col<T>(Q, choice.variant, choice.rpl, s, views, vt, proj, accumulate, nviews,
-                  (unsigned)vt_bytes);
+  dispatch_col<T>(Q, choice, s, views, vt, proj, accumulate, nviews, (unsigned)vt_bytes);
   cbct_prof_mark(ctx, PROF_FP, 1, s);
   CBCT_LAUNCH_CHECK(ctx, "k_fp_col");
   return CBCT_OK;
@@ -1252,17 +1280,19 @@ int cbct_fp_autotune(cbct_ctx ctx, const cbct_geom *g, int view0, int nviews, in
   const FPChoice heuristic = select_variant(ctx, g, P, view0, nviews, esz, spp);
   ctx->fp_engine = saved_engine;
   if (heuristic.variant == 0) return CBCT_OK;   // the column engines do not apply
-  // candidates: the heuristic's; the cached variants with 2- and 3-chunk
-  // windows at several tiles; the per-step variant of the storage type
+  // candidates: the heuristic's; the cached variants at several tiles with the
+  // windows they need; the per-step variant of the storage type
   std::vector<FPChoice> cand{heuristic};
-  auto add = [&](int v, int r) {
+  auto add = [&](int v, int r, int zc) {
     for (auto &c : cand)
-      if (c.variant == v && c.rpl == r) return;
-    cand.push_back({v, r});
+      if (c.variant == v && c.rpl == r && c.zc == zc) return;
+    cand.push_back({v, r, zc});
   };
-  for (int m : {4, 6, 8, 12}) add(3, rows_per_lane(P.nv, m));
-  for (int m : {6, 8}) add(4, rows_per_lane(P.nv, m));
-  add(esz == 2 ? 2 : 1, rows_per_lane(P.nv, 8));
+  for (int m : {2, 4, 6, 8, 12}) {
+    const int rpl = rows_per_lane(P.nv, m), zc = window_zc(ctx, g, P.nv, rpl, view0, nviews);
+    if (zc <= FP_ZC_MAX) add(3, rpl, zc);
+  }
+  add(esz == 2 ? 2 : 1, rows_per_lane(P.nv, 8), 0);
   // scratch volume and projections (contents do not change the timing)
   const size_t nvox = (size_t)g->nx * g->ny * g->nz;
   const size_t nproj = (size_t)g->nu * g->nv * (size_t)nviews;
@@ -1285,6 +1315,7 @@ int cbct_fp_autotune(cbct_ctx ctx, const cbct_geom *g, int view0, int nviews, in
   auto trial = [&](const FPChoice &c) {
     ctx->fp_force_variant = c.variant;
     ctx->fp_force_rpl = c.rpl;
+    ctx->fp_force_zc = c.zc;
     ctx->fp_force_vg = c.vg;
     double t = 1e300;
     for (int rep = 0; rep < 3 && rc == CBCT_OK; ++rep) {   // first run warms up
@@ -1306,9 +1337,10 @@ int cbct_fp_autotune(cbct_ctx ctx, const cbct_geom *g, int view0, int nviews, in
   for (size_t c = 0; c < cand.size() && rc == CBCT_OK; ++c) trial(cand[c]);
   const FPChoice base = best;
   for (int vg : {1, 3, 6, 8})
-    if (rc == CBCT_OK && vg != ctx->fp_view_group) trial({base.variant, base.rpl, vg});
+    if (rc == CBCT_OK && vg != ctx->fp_view_group) trial({base.variant, base.rpl, base.zc, vg});
   ctx->fp_force_variant = 0;
   ctx->fp_force_rpl = 0;
+  ctx->fp_force_zc = 0;
   ctx->fp_force_vg = 0;
   (void)hipStreamSynchronize(s);
   (void)hipEventDestroy(e0);
@@ -1355,7 +1387,7 @@ const char *cbct_fp_kernel(cbct_ctx ctx, const cbct_geom *g, int view0, int nvie
   if (make_params(ctx, g, spp, P)) return "";
   const size_t esz = (dtype == CBCT_BF16 || ctx->work_dtype == CBCT_BF16) ? 2 : 4;
   const int v = select_variant(ctx, g, P, view0, nviews, esz, spp).variant;
-  return v == 0 ? "k_fp_ray" : v >= 3 ? "k_fp_colc" : "k_fp_col";
+  return v == 0 ? "k_fp_ray" : v == 3 ? "k_fp_colc" : "k_fp_col";
 }
 
 }  // extern "C"

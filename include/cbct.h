@@ -135,12 +135,12 @@ int cbct_bp(cbct_ctx ctx, const cbct_geom *g, int view0, int nviews, const void 
 
 /* Forward-projector engine: 1 = detector-column sharing (default; one wave per
  * detector column interpolates the shared z-line once per step: the variant
- * that keeps the column's four corner z-lines in registers across steps when
- * every row group's z window fits two chunks of 128 z, else the per-step
- * variant measured fastest for the storage type), 2 = the other per-step
- * variant, 3 / 4 = the cached variant with a two / three chunk window (falls
- * back to per-step loads per column when the window is larger), 0 = one
- * thread per ray.  All give bitwise-identical projections.  No reference
+ * that keeps the column's four corner z-lines in registers across steps, with
+ * the tile and the z window (64 to 384 z) that cost least for the geometry,
+ * when a row group's z window fits 384 z, else the per-step variant measured
+ * fastest for the storage type), 2 = the other per-step variant, 3 / 4 = the
+ * cached variant with a window of 256 / 384 z (falls back to per-step loads per
+ * column when the window is larger), 0 = one thread per ray.  All give bitwise-identical projections.  No reference
  * counterpart (the reference has one texture-based kernel). */
 int cbct_fp_engine(cbct_ctx ctx, int engine);
 
@@ -165,8 +165,9 @@ const char *cbct_fp_kernel(cbct_ctx ctx, const cbct_geom *g, int view0, int nvie
                            int vol_dtype, float samples_per_pixel);
 
 /* Column-engine tile: the most detector rows one lane carries (1..12,
- * default 8).  Columns with more rows than 64 x this are split into row
- * groups, each with its own z-line loads.  Results do not depend on it.  No
+ * default 8; engine 1 chooses up to 12 by itself until this is called).
+ * Columns with more rows than 64 x this are split into row groups, each with
+ * its own z-line loads.  Results do not depend on it.  No
  * reference counterpart. */
 int cbct_fp_tile(cbct_ctx ctx, int max_rows_per_lane);
 

@@ -5,7 +5,11 @@ single-pass bound of the other parity tests).
 Clipped rays: rays leaving through the top or bottom are taken 8 samples x 8
 rays at a time, so sample counts off the multiples of 8, row blocks with a few
 clipped rays, blocks of 64 rows that end ragged, and odd z for the BF16 pairs
-are where it can go wrong."""
+are where it can go wrong.
+
+Cached z windows: 64 to 384 z in pieces of several widths, chosen by the z
+range that a row group's rays cross; volume heights on both sides of every
+width, ragged row counts and up to 12 rows per lane."""
 import numpy as np
 import pytest
 
@@ -54,6 +58,32 @@ def test_clipped_rays(ctx, case, dtype):
         v = v.to(torch.bfloat16)
     ctx.set_views(angles, offsets)
     a, b = project(ctx, g, v, 5, 0), project(ctx, g, v, 5, 1)
+    assert torch.equal(a, b)
+    ref = O.fp(to_oracle(g), angles, offsets, v.double().cpu().numpy())
+    assert rel_l2(b.cpu().numpy(), ref) <= TOL
+
+
+# (nz, nv): the window grows with nz; 12 rows per lane at most
+WINDOWS = [(1, 1), (50, 64), (57, 65), (60, 130), (118, 129), (122, 300), (180, 257), (186, 383), (245, 320),
+           (251, 449), (310, 512), (314, 577), (372, 700), (378, 768), (420, 768)]
+
+
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+@pytest.mark.parametrize("case", WINDOWS)
+def test_z_windows(ctx, case, dtype):
+    nz, nv = case
+    # magnification 1.5: the detector sees the whole height and no more, so the
+    # rays cross the window's whole width
+    g = geom(9, 7, nz, 6, nv, fov=(20.0, 1.48 * nz))
+    angles = angles_full(7)
+    offsets = np.tile(np.array([[0.2, 0.3]], np.float32), (7, 1))
+    print("CASE window", case, dtype, flush=True)
+    vol = np.random.default_rng(nz).random((nz, 7, 9)) + 0.1
+    v = torch.from_numpy(vol.astype(np.float32)).cuda()
+    if dtype == "bf16":
+        v = v.to(torch.bfloat16)
+    ctx.set_views(angles, offsets)
+    a, b = project(ctx, g, v, 7, 0), project(ctx, g, v, 7, 1)
     assert torch.equal(a, b)
     ref = O.fp(to_oracle(g), angles, offsets, v.double().cpu().numpy())
     assert rel_l2(b.cpu().numpy(), ref) <= TOL
