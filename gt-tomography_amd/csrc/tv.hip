@@ -37,11 +37,11 @@ struct Grad {
 // FMA residual (Markstein 1990), which gives the correctly rounded quotients
 // but for rare last bits; the compiler's own sequences scale and fix up
 // exponents that cannot occur here (52 against 29 instructions per gradient).
-// Norms from 2^50 on, infinities and NaN take the plain operations.
+// Norms whose square overflows, infinities and NaN take the plain operations.
 __device__ __forceinline__ Grad tv_grad(float c, float cx, float cy, float cz, float scale) {
   const float g0 = (cx - c) * scale, g1 = (cy - c) * scale, g2 = (cz - c) * scale;
   const float a = g0 * g0 + g1 * g1 + g2 * g2;
-  if (!(a < 0x1p100f)) {
+  if (!(a < INFINITY)) {
     const float den = fmaxf(1.0f, sqrtf(a));
     return {g0 / den, g1 / den, g2 / den};
   }

@@ -28,8 +28,8 @@ SHAPES = [(1, 1, 1), (2, 1, 64), (1, 2, 65), (3, 3, 63), (5, 8, 130), (4, 9, 1),
 @pytest.mark.parametrize("scale", [1.0, 1e12, 1e17, 1e-30])
 @pytest.mark.parametrize("shape", SHAPES)
 def test_tv_tiles(ctx, shape, scale):
-    """scale 1e12: norms far above one; 1e17: norms from 2^50 on (plain
-    operations); 1e-30: gradients far below one, passed through."""
+    """scale 1e12: norms far above one; 1e17: their squares near the largest
+    float; 1e-30: gradients far below one, passed through."""
     print("CASE tv", shape, scale, flush=True)
     rng = np.random.default_rng(abs(hash(shape)) % 1000)
     x = (rng.random(shape) * scale).astype(np.float32)
