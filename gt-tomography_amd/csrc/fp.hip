@@ -75,20 +75,26 @@ __device__ __forceinline__ float ld<unsigned short>(const unsigned short *p, uns
   return bf16_to_f32(p[i]);
 }
 
-// Column part of the ray setup (shared by every ray with detector column i).
+// Ray setup in FP64.  Every engine takes its parameters from these functions,
+// and only the explicit fma calls fuse, so that the same ray has the same bits
+// whatever surrounds the call.
+
+// Column part (shared by every ray with detector column i).
 struct ColSetup {
-  double S0, S1, d0, d1, lo, hi;  // lo/hi: slab limits from the x and y faces
+  double S0, S1, d0, d1, dd, lo, hi;  // dd: d0^2 + d1^2; lo/hi: slab limits from the x and y faces
 };
 
 __device__ __forceinline__ ColSetup col_setup(const FPParams &P, const ViewD &vw, int i) {
+#pragma clang fp contract(off)
   ColSetup C;
   const double c = vw.c, s = vw.s;
   C.S0 = s * P.sad;  // R(theta) (0,-SAD,0)
   C.S1 = -c * P.sad;
-  const double pu = ((i + 0.5) / P.nu - 0.5) * P.fu + vw.off_u;
+  const double pu = fma((i + 0.5) / P.nu - 0.5, P.fu, vw.off_u);
   const double add = P.sdd - P.sad;
-  C.d0 = (c * pu - s * add) - C.S0;
-  C.d1 = (s * pu + c * add) - C.S1;
+  C.d0 = fma(c, pu, -(s * add)) - C.S0;
+  C.d1 = fma(s, pu, c * add) - C.S1;
+  C.dd = fma(C.d1, C.d1, C.d0 * C.d0);
   const double hx = P.lx * 0.5, hy = P.ly * 0.5;
   double tA = (hx - C.S0) / C.d0, tB = (-hx - C.S0) / C.d0;
   C.lo = fmin(tB, tA);
@@ -100,33 +106,47 @@ __device__ __forceinline__ ColSetup col_setup(const FPParams &P, const ViewD &vw
   return C;
 }
 
+// Detector height of row j.
+__device__ __forceinline__ double row_height(const FPParams &P, const ViewD &vw, int j) {
+#pragma clang fp contract(off)
+  return fma((j + 0.5) / P.nv - 0.5, P.fv, vw.off_v);
+}
+
+// Start, increment (in texel space: normalised * N - 0.5, plus 1 for the leading
+// zero border) and step length of the n samples on [a1, a2]; span = a2 - a1, h =
+// span / n.  The x/y part does not depend on the row.
+__device__ __forceinline__ void ray_xy(const FPParams &P, const ColSetup &C, double a1, double h,
+                                       float &px, float &qx, float &py, float &qy) {
+#pragma clang fp contract(off)
+  px = (float)fma(fma(a1, C.d0, C.S0) / P.lx + 0.5, (double)P.nx, 0.5);
+  py = (float)fma(fma(a1, C.d1, C.S1) / P.ly + 0.5, (double)P.ny, 0.5);
+  qx = (float)(C.d0 / P.lx * h * P.nx);
+  qy = (float)(C.d1 / P.ly * h * P.ny);
+}
+__device__ __forceinline__ void ray_z(const FPParams &P, const ColSetup &C, double d2, double a1,
+                                      double span, double h, float &pz, float &qz, float &step) {
+#pragma clang fp contract(off)
+  pz = (float)fma((a1 * d2) / P.lz + 0.5, (double)P.nz, 0.5);
+  qz = (float)(d2 / P.lz * h * P.nz);
+  step = (float)(sqrt(fma(d2, d2, C.dd)) * fabs(span) / P.n);
+}
+
 struct RaySetup {
-  double a1, a2;
   float p[3], q[3], step;
 };
 
-// Per-ray completion of the setup (row j).
+// Row j's ray of the column: clipped to the z slab [-t, t], sampled.
 __device__ __forceinline__ RaySetup ray_finish(const FPParams &P, const ViewD &vw,
                                                const ColSetup &C, int j) {
+#pragma clang fp contract(off)
   RaySetup R;
-  const double pv = ((j + 0.5) / P.nv - 0.5) * P.fv + vw.off_v;
-  const double d2 = pv;
-  const double hz = P.lz * 0.5;
-  const double tA = hz / d2, tB = -hz / d2;
-  const double lo = fmax(C.lo, fmin(tB, tA));
-  const double hi = fmin(C.hi, fmax(tB, tA));
-  R.a1 = fmax(lo, 0.0);
-  R.a2 = fmin(hi, 1.0);
-  const double span = R.a2 - R.a1;
-  const double h = span / P.n;
-  R.step = (float)(sqrt(C.d0 * C.d0 + C.d1 * C.d1 + d2 * d2) * fabs(span) / P.n);
-  // texel = normalised*N - 0.5, plus 1 for the leading zero border
-  R.p[0] = (float)(((C.S0 + R.a1 * C.d0) / P.lx + 0.5) * P.nx + 0.5);
-  R.p[1] = (float)(((C.S1 + R.a1 * C.d1) / P.ly + 0.5) * P.ny + 0.5);
-  R.p[2] = (float)(((R.a1 * d2) / P.lz + 0.5) * P.nz + 0.5);
-  R.q[0] = (float)(C.d0 / P.lx * h * P.nx);
-  R.q[1] = (float)(C.d1 / P.ly * h * P.ny);
-  R.q[2] = (float)(d2 / P.lz * h * P.nz);
+  const double d2 = row_height(P, vw, j);
+  const double t = fabs(P.lz * 0.5 / d2);
+  const double a1 = fmax(fmax(C.lo, -t), 0.0);
+  const double a2 = fmin(fmin(C.hi, t), 1.0);
+  const double span = a2 - a1, h = span / P.n;
+  ray_xy(P, C, a1, h, R.p[0], R.q[0], R.p[1], R.q[1]);
+  ray_z(P, C, d2, a1, span, h, R.p[2], R.q[2], R.step);
   return R;
 }
 
@@ -341,6 +361,18 @@ struct Cell {
     else if (t == Z - 1 && ONE) return __uint_as_float(w[c][WORDS - 1] << 16);
     else return __uint_as_float(t & 1 ? w[c][t >> 1] & 0xffff0000u : w[c][t >> 1] << 16);
   }
+  // the bilinear z-line at weights (ax, ay) into LDS
+  __device__ __forceinline__ void combine(float *zl, int lane, float ax, float ay) const {
+    float o[Z];
+#pragma unroll
+    for (int t = 0; t < Z; ++t) {
+      const float v00 = at(0, t), v01 = at(2, t);
+      const float c0 = fmaf(ax, at(1, t) - v00, v00);
+      const float c1 = fmaf(ax, at(3, t) - v01, v01);
+      o[t] = fmaf(ay, c1 - c0, c0);
+    }
+    store(zl, lane, o);
+  }
   // a lane's Z values to their places of the z-line in LDS
   static __device__ __forceinline__ void store(float *zl, int lane, const float (&o)[Z]) {
     int k = 0;
@@ -501,7 +533,7 @@ __device__ __forceinline__ void col_block(const FPParams &P, unsigned W, unsigne
 //     step's cell right after this step's combine.  Every load fetches the
 //     whole window; z past the part a step needs are never read.
 // All produce the same bits as the per-ray engine.
-template <typename T, int RPL, bool SSTEP, int ZP, int ZC>
+template <typename T, int RPL, bool SSTEP, int ZP, int ZC, int D>
 __device__ __forceinline__ void fp_col_body(const FPParams &P, const ViewD *__restrict__ views,
                                             const T *__restrict__ vt, float *__restrict__ proj,
                                             int accumulate, unsigned ngroups, unsigned nblocks,
@@ -523,22 +555,17 @@ __device__ __forceinline__ void fp_col_body(const FPParams &P, const ViewD *__re
     const double a1c = fmax(C.lo, 0.0);
     const double a2c = fmin(C.hi, 1.0);
     const bool col_ok = (a2c - a1c) >= 0.0;   // h >= 0 keeps tz monotone in the row
-    // the expressions of ray_finish for the shared (a1, a2), x/y once per column
+    // the shared (a1, a2): x/y once per column, z per row
     const double span = a2c - a1c, h = span / P.n;
-    px0 = (float)(((C.S0 + a1c * C.d0) / P.lx + 0.5) * P.nx + 0.5);
-    py0 = (float)(((C.S1 + a1c * C.d1) / P.ly + 0.5) * P.ny + 0.5);
-    qx = (float)(C.d0 / P.lx * h * P.nx);
-    qy = (float)(C.d1 / P.ly * h * P.ny);
+    ray_xy(P, C, a1c, h, px0, qx, py0, qy);
     int jmin = 0x7fffffff, jmax = -1;
 #pragma unroll
     for (int r = 0; r < RPL; ++r) {
       const int j = row0 + r * 64 + lane;
       acc[r] = 0.0f;
-      const double d2 = ((j + 0.5) / P.nv - 0.5) * P.fv + vw.off_v;
+      const double d2 = row_height(P, vw, j);
       const double t = fabs(P.lz * 0.5 / d2);   // the z slab is [-t, t]
-      pz[r] = (float)(((a1c * d2) / P.lz + 0.5) * P.nz + 0.5);
-      qz[r] = (float)(d2 / P.lz * h * P.nz);
-      stp[64 * r] = (float)(sqrt(C.d0 * C.d0 + C.d1 * C.d1 + d2 * d2) * fabs(span) / P.n);
+      ray_z(P, C, d2, a1c, span, h, pz[r], qz[r], stp[64 * r]);
       if (j < P.nv) {
         valid_mask |= 1u << r;
         if (col_ok && fmax(fmax(C.lo, -t), 0.0) == a1c && fmin(fmin(C.hi, t), 1.0) == a2c) {
@@ -606,79 +633,116 @@ __device__ __forceinline__ void fp_col_body(const FPParams &P, const ViewD *__re
       // (cell coordinates are packed as two 16-bit halves below)
       if (zhi_max - zb0 < 64 * ZC && P.cx < 65535.0f && P.cy < 65535.0f) {
         done = true;
-        Cell<T, ZC> L;
-        L.setup(lane, so_x);
         const unsigned zoff = (unsigned)zb0 * esz;
-        const float *zb = zl - zb0;
-        // all four lines of cell (ix, iy)
-        auto load_cell = [&](int ix, int iy) __attribute__((always_inline)) {
-          L.load(rsrc, lane, ((unsigned)iy * P.px + (unsigned)ix) * PZ * esz + zoff, so_x, so_y);
+        // byte offset of cell (c & 0xffff, c >> 16)'s line 00 at the window
+        auto cell_base = [&](unsigned c) __attribute__((always_inline)) {
+          return ((c >> 16) * P.px + (c & 0xffffu)) * PZ * esz + zoff;
         };
-        // the combined z-line of the cell's lines into LDS
-        auto combine = [&](const float ax, const float ay) __attribute__((always_inline)) {
-          float o[ZC];
+        // x/y position of step m, the same for the whole wave
+        auto step_x = [&](float fm) { return __builtin_amdgcn_fmed3f(fmaf(fm, qx, px0), 0.0f, P.cx); };
+        auto step_y = [&](float fm) { return __builtin_amdgcn_fmed3f(fmaf(fm, qy, py0), 0.0f, P.cy); };
+        auto step_cell = [&](float fm) { return (unsigned)step_x(fm) | ((unsigned)step_y(fm) << 16); };
+        if constexpr (D > 1) {
+          // Few waves: the step's own latencies (lines from L2, the z-line
+          // through LDS) are not hidden by other waves but by the steps
+          // around it.  The lines of D steps are in flight, each step's reloaded
+          // for D steps on once its combine has used them, and a step's reads
+          // of its z-line (two buffers) return during the next step's combine.
+          Cell<T, ZC> S[D];
+          float pa[RPL], pb[RPL], paz[RPL];   // the last step's reads
 #pragma unroll
-          for (int t = 0; t < ZC; ++t) {
-            const float v00 = L.at(0, t), v01 = L.at(2, t);
-            const float c0 = fmaf(ax, L.at(1, t) - v00, v00);
-            const float c1 = fmaf(ax, L.at(3, t) - v01, v01);
-            o[t] = fmaf(ay, c1 - c0, c0);
+          for (int r = 0; r < RPL; ++r) pa[r] = pb[r] = paz[r] = 0.0f;   // adds 0 before step 0
+          const int last = P.n - 1;
+          const unsigned c0 = step_cell((float)min(lane, last));
+#pragma unroll
+          for (int d = 0; d < D; ++d) {
+            S[d].setup(lane, so_x);
+            S[d].load(rsrc, lane, cell_base((unsigned)__builtin_amdgcn_readlane((int)c0, d)), so_x, so_y);
           }
-          L.store(zl, lane, o);
-          wave_lds_sync();
-        };
-        // every ray's z-lerp from the combined z-line
-        auto rays = [&](const float fm) __attribute__((always_inline)) {
+          auto finish = [&]() __attribute__((always_inline)) {
 #pragma unroll
-            for (int r = 0; r < RPL; ++r) {
-              const float tz = fmaf(fm, qz[r], pz[r]);  // in [0, nz+1]: checked above
-              const int iz = (int)tz;
-              const float az = __builtin_amdgcn_fractf(tz);
-              const float a = zb[iz], b = zb[iz + 1];
-              acc[r] += fmaf(az, b - a, a);
+            for (int r = 0; r < RPL; ++r) acc[r] += fmaf(paz[r], pb[r] - pa[r], pa[r]);
+          };
+          for (int mb = 0; mb < P.n; mb += 64) {
+            const float fml = (float)(mb + lane);
+            const int axl = __float_as_int(__builtin_amdgcn_fractf(step_x(fml)));
+            const int ayl = __float_as_int(__builtin_amdgcn_fractf(step_y(fml)));
+            const int cn = (int)step_cell((float)min(mb + lane + D, last));   // D steps on
+            const int cnt = __builtin_amdgcn_readfirstlane(min(64, P.n - mb));
+            for (int l = 0; l < cnt; l += D) {
+#pragma unroll
+              for (int d = 0; d < D; ++d) {
+                if (l + d >= cnt) break;
+                float *z = zl + (d & 1) * 64 * ZC;
+                S[d].fix();
+                S[d].combine(z, lane, __int_as_float(__builtin_amdgcn_readlane(axl, l + d)),
+                             __int_as_float(__builtin_amdgcn_readlane(ayl, l + d)));
+                S[d].load(rsrc, lane, cell_base((unsigned)__builtin_amdgcn_readlane(cn, l + d)), so_x, so_y);
+                finish();
+                wave_lds_sync();
+                const float fm = (float)(mb + l + d);
+                const float *zr = z - zb0;
+#pragma unroll
+                for (int r = 0; r < RPL; ++r) {
+                  const float tz = fmaf(fm, qz[r], pz[r]);
+                  const int iz = (int)tz;
+                  paz[r] = __builtin_amdgcn_fractf(tz);
+                  pa[r] = zr[iz];
+                  pb[r] = zr[iz + 1];
+                }
+                wave_lds_sync();
+              }
             }
-            wave_lds_sync();
-        };
-        // The x/y part of a step, the same for the whole wave, is evaluated for
-        // 64 steps at once, step mb + lane in each lane (the same expressions
-        // as per step, so the same values), and each step reads its cell and
-        // weights back into scalar registers.  The lines of the next step's
-        // cell, when it changes, are all four reloaded straight into their
-        // registers once this step's combine has used them, so they arrive
-        // while this step's rays run.  Keeping the lines that the two cells
-        // share saves half the bytes, but the register moves wait on the loads:
-        // 13.1 against 12.6 ms (FP32 copies, 512^3, 48 views).
-        const float s0x = __builtin_amdgcn_fmed3f(fmaf(0.0f, qx, px0), 0.0f, P.cx);
-        const float s0y = __builtin_amdgcn_fmed3f(fmaf(0.0f, qy, py0), 0.0f, P.cy);
-        int cx = __builtin_amdgcn_readfirstlane((int)s0x), cy = __builtin_amdgcn_readfirstlane((int)s0y);
-        load_cell(cx, cy);
-        bool fresh = true;   // loaded and not yet fixed
-        for (int mb = 0; mb < P.n; mb += 64) {
-          const float fml = (float)(mb + lane);
-          const float sxl = __builtin_amdgcn_fmed3f(fmaf(fml, qx, px0), 0.0f, P.cx);
-          const float syl = __builtin_amdgcn_fmed3f(fmaf(fml, qy, py0), 0.0f, P.cy);
-          const int axl = __float_as_int(__builtin_amdgcn_fractf(sxl));
-          const int ayl = __float_as_int(__builtin_amdgcn_fractf(syl));
-          // cell of step mb + lane + 1 (the next step's)
-          const float fmn = (float)(mb + lane + 1);
-          const float sxn = __builtin_amdgcn_fmed3f(fmaf(fmn, qx, px0), 0.0f, P.cx);
-          const float syn = __builtin_amdgcn_fmed3f(fmaf(fmn, qy, py0), 0.0f, P.cy);
-          const int cn = (int)((unsigned)sxn | ((unsigned)syn << 16));
-          const int cnt = __builtin_amdgcn_readfirstlane(min(64, P.n - mb));
-          for (int l = 0; l < cnt; ++l) {
-            const float ax = __int_as_float(__builtin_amdgcn_readlane(axl, l));
-            const float ay = __int_as_float(__builtin_amdgcn_readlane(ayl, l));
-            if (fresh) L.fix();
-            combine(ax, ay);
-            const unsigned c = (unsigned)__builtin_amdgcn_readlane(cn, l);
-            const int nx = (int)(c & 0xffffu), ny = (int)(c >> 16);
-            fresh = mb + l + 1 < P.n && (nx != cx || ny != cy);
-            if (fresh) {
-              load_cell(nx, ny);
-              cx = nx;
-              cy = ny;
+          }
+          finish();
+        } else {
+          Cell<T, ZC> L;
+          L.setup(lane, so_x);
+          const float *zb = zl - zb0;
+          // every ray's z-lerp from the combined z-line
+          auto rays = [&](const float fm) __attribute__((always_inline)) {
+#pragma unroll
+              for (int r = 0; r < RPL; ++r) {
+                const float tz = fmaf(fm, qz[r], pz[r]);  // in [0, nz+1]: checked above
+                const int iz = (int)tz;
+                const float az = __builtin_amdgcn_fractf(tz);
+                const float a = zb[iz], b = zb[iz + 1];
+                acc[r] += fmaf(az, b - a, a);
+              }
+              wave_lds_sync();
+          };
+          // The x/y part of a step, the same for the whole wave, is evaluated for
+          // 64 steps at once, step mb + lane in each lane (the same expressions
+          // as per step, so the same values), and each step reads its cell and
+          // weights back into scalar registers.  The lines of the next step's
+          // cell, when it changes, are all four reloaded straight into their
+          // registers once this step's combine has used them, so they arrive
+          // while this step's rays run.  Keeping the lines that the two cells
+          // share saves half the bytes, but the register moves wait on the loads:
+          // 13.1 against 12.6 ms (FP32 copies, 512^3, 48 views).
+          unsigned cur = (unsigned)__builtin_amdgcn_readfirstlane((int)step_cell(0.0f));
+          L.load(rsrc, lane, cell_base(cur), so_x, so_y);
+          bool fresh = true;   // loaded and not yet fixed
+          for (int mb = 0; mb < P.n; mb += 64) {
+            const float fml = (float)(mb + lane);
+            const int axl = __float_as_int(__builtin_amdgcn_fractf(step_x(fml)));
+            const int ayl = __float_as_int(__builtin_amdgcn_fractf(step_y(fml)));
+            const int cn = (int)step_cell((float)(mb + lane + 1));   // the next step's
+            const int cnt = __builtin_amdgcn_readfirstlane(min(64, P.n - mb));
+            for (int l = 0; l < cnt; ++l) {
+              const float ax = __int_as_float(__builtin_amdgcn_readlane(axl, l));
+              const float ay = __int_as_float(__builtin_amdgcn_readlane(ayl, l));
+              if (fresh) L.fix();
+              L.combine(zl, lane, ax, ay);
+              wave_lds_sync();
+              const unsigned nxt = (unsigned)__builtin_amdgcn_readlane(cn, l);
+              fresh = mb + l + 1 < P.n && nxt != cur;
+              if (fresh) {
+                L.load(rsrc, lane, cell_base(nxt), so_x, so_y);
+                cur = nxt;
+              }
+              rays((float)(mb + l));
             }
-            rays((float)(mb + l));
           }
         }
       }
@@ -834,7 +898,7 @@ __global__ void __launch_bounds__(64) k_fp_col(FPParams P, const ViewD *__restri
                                                const T *__restrict__ vt, float *__restrict__ proj,
                                                int accumulate, unsigned ngroups, unsigned nblocks,
                                                unsigned vt_bytes) {
-  fp_col_body<T, RPL, SSTEP, ZP, 0>(P, views, vt, proj, accumulate, ngroups, nblocks, vt_bytes);
+  fp_col_body<T, RPL, SSTEP, ZP, 0, 1>(P, views, vt, proj, accumulate, ngroups, nblocks, vt_bytes);
 }
 
 // The cached variant, held to five waves per SIMD, four from 8 rows per lane on
@@ -842,13 +906,13 @@ __global__ void __launch_bounds__(64) k_fp_col(FPParams P, const ViewD *__restri
 // six / seven waves 12.8 / 12.8 / 14.1 / 15.2 ms (FP32 copies), 11.0 / 11.1 /
 // 11.2 / 12.3 (BF16); 291^3, 32 views, 8 rows: 1.61 / 1.70 / 2.03 / 2.19 and
 // 1.49 / 1.57 / 1.63 / 1.82.
-constexpr int colc_waves(int rpl) { return rpl >= 8 ? 4 : 5; }
-template <typename T, int RPL, int ZC>
-__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(colc_waves(RPL))))
+constexpr int colc_waves(int rpl, int d) { return d > 1 ? 2 : rpl >= 8 ? 4 : 5; }
+template <typename T, int RPL, int ZC, int D>
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(colc_waves(RPL, D))))
 k_fp_colc(FPParams P, const ViewD *__restrict__ views, const T *__restrict__ vt,
           float *__restrict__ proj, int accumulate, unsigned ngroups, unsigned nblocks,
           unsigned vt_bytes) {
-  fp_col_body<T, RPL, true, 2, ZC>(P, views, vt, proj, accumulate, ngroups, nblocks, vt_bytes);
+  fp_col_body<T, RPL, true, 2, ZC, D>(P, views, vt, proj, accumulate, ngroups, nblocks, vt_bytes);
 }
 
 // ------------------------------------------------------------ layouts
@@ -976,7 +1040,7 @@ int make_params(cbct_ctx ctx, const cbct_geom *g, float spp, FPParams &P) {
   return CBCT_OK;
 }
 
-template <typename T, int RPL, bool SSTEP, int ZP, int ZC>
+template <typename T, int RPL, bool SSTEP, int ZP, int ZC, int D = 1>
 void launch_col(const FPParams &P, hipStream_t s, const ViewD *views, const T *vt, float *proj,
                 int acc, int nviews, unsigned vt_bytes) {
   const unsigned ngroups = (unsigned)((P.nv + 64 * RPL - 1) / (64 * RPL));
@@ -997,7 +1061,7 @@ void launch_col(const FPParams &P, hipStream_t s, const ViewD *views, const T *v
     const ViewD *vw = views + v0;
     float *pj = proj + (size_t)v0 * P.nu * P.nv;
     if constexpr (ZC > 0)
-      hipLaunchKernelGGL((k_fp_colc<T, RPL, ZC>), dim3(nblocks), dim3(64), lds, s, Q, vw, vt, pj, acc,
+      hipLaunchKernelGGL((k_fp_colc<T, RPL, ZC, D>), dim3(nblocks), dim3(64), lds, s, Q, vw, vt, pj, acc,
                          ngroups, nblocks, vt_bytes);
     else
       hipLaunchKernelGGL((k_fp_col<T, RPL, SSTEP, ZP>), dim3(nblocks), dim3(64), lds, s, Q, vw, vt, pj,
@@ -1014,13 +1078,25 @@ struct FPChoice {
   int rpl;      // rows per lane
   int zc = 0;
   int vg = 0;   // views per launch group; 0 = the context's setting
+  bool deep = false;   // cached variant with the lines of four steps in flight
 };
+// Deep variants: windows of 64 and 128 z, up to 4 rows per lane, for launches
+// of fewer waves than hide each other's latencies (8 per SIMD).  64^3, 9 views
+// (864 waves) 40 -> 31 us with the padded copy, 96^3, 10 views (1500) 61 -> 51,
+// 128^3, 24 views (6144) 136 -> 125; from 12288 waves on they cost 2-9%, and
+// with wider windows they gain nothing.
+constexpr int FP_DEEP_RPL = 4, FP_DEEP_ZC = 2;
+constexpr size_t FP_DEEP_WAVES = 8192;
 
 template <typename T, int RPL>
 void launch_col_w(const FPParams &P, const FPChoice &c, hipStream_t s, const ViewD *views, const T *vt,
                   float *proj, int acc, int nviews, unsigned vt_bytes) {
   if (c.variant == 1) return launch_col<T, RPL, false, 1, 0>(P, s, views, vt, proj, acc, nviews, vt_bytes);
   if (c.variant == 2) return launch_col<T, RPL, true, 2, 0>(P, s, views, vt, proj, acc, nviews, vt_bytes);
+  if constexpr (RPL <= FP_DEEP_RPL) {
+    if (c.deep && c.zc == 1) return launch_col<T, RPL, true, 2, 1, 4>(P, s, views, vt, proj, acc, nviews, vt_bytes);
+    if (c.deep && c.zc == 2) return launch_col<T, RPL, true, 2, 2, 4>(P, s, views, vt, proj, acc, nviews, vt_bytes);
+  }
   switch (c.zc) {
     case 1: launch_col<T, RPL, true, 2, 1>(P, s, views, vt, proj, acc, nviews, vt_bytes); break;
     case 2: launch_col<T, RPL, true, 2, 2>(P, s, views, vt, proj, acc, nviews, vt_bytes); break;
@@ -1123,6 +1199,8 @@ FPChoice default_variant(cbct_ctx ctx, const cbct_geom *g, const FPParams &P, in
     if (zc <= FP_ZC_MAX && cost < best_cost) {
       best_cost = cost;
       best = {3, rpl, zc};
+      best.deep = zc <= FP_DEEP_ZC && rpl <= FP_DEEP_RPL &&
+                  (size_t)groups * P.nu * nviews < FP_DEEP_WAVES;
     }
   }
   return best;

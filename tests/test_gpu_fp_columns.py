@@ -68,22 +68,27 @@ WINDOWS = [(1, 1), (50, 64), (57, 65), (60, 130), (118, 129), (122, 300), (180, 
            (251, 449), (310, 512), (314, 577), (372, 700), (378, 768), (420, 768)]
 
 
+# launches of 8192 waves (detector columns x row groups x views) and more leave
+# the variant that keeps several steps in flight; the last one is just below
+MANY = [(1, 1, 70, 118), (50, 64, 64, 128), (118, 129, 70, 120), (60, 130, 66, 125), (122, 240, 127, 64)]
+
+
 @pytest.mark.parametrize("dtype", ["f32", "bf16"])
-@pytest.mark.parametrize("case", WINDOWS)
+@pytest.mark.parametrize("case", [w + (6, 7) for w in WINDOWS] + MANY)
 def test_z_windows(ctx, case, dtype):
-    nz, nv = case
+    nz, nv, nu, nviews = case
     # magnification 1.5: the detector sees the whole height and no more, so the
     # rays cross the window's whole width
-    g = geom(9, 7, nz, 6, nv, fov=(20.0, 1.48 * nz))
-    angles = angles_full(7)
-    offsets = np.tile(np.array([[0.2, 0.3]], np.float32), (7, 1))
+    g = geom(9, 7, nz, nu, nv, fov=(20.0, 1.48 * nz))
+    angles = angles_full(nviews)
+    offsets = np.tile(np.array([[0.2, 0.3]], np.float32), (nviews, 1))
     print("CASE window", case, dtype, flush=True)
     vol = np.random.default_rng(nz).random((nz, 7, 9)) + 0.1
     v = torch.from_numpy(vol.astype(np.float32)).cuda()
     if dtype == "bf16":
         v = v.to(torch.bfloat16)
     ctx.set_views(angles, offsets)
-    a, b = project(ctx, g, v, 7, 0), project(ctx, g, v, 7, 1)
+    a, b = project(ctx, g, v, nviews, 0), project(ctx, g, v, nviews, 1)
     assert torch.equal(a, b)
     ref = O.fp(to_oracle(g), angles, offsets, v.double().cpu().numpy())
     assert rel_l2(b.cpu().numpy(), ref) <= TOL
