@@ -33,6 +33,7 @@ struct DeviceBuffer {
 struct Workspace {
   int device = 0;
   DeviceBuffer vol_pad;     // padded / repacked volume for the forward projector
+  DeviceBuffer vol_cells;   // forward projector: packed (x, y) corners of the volume copy
   DeviceBuffer proj_pad;    // padded projections for the backprojector
   DeviceBuffer red;         // reduction partials
   DeviceBuffer filt_tmp;    // filter staging

@@ -73,7 +73,7 @@ int cbct_check_geom(cbct_ctx ctx, const cbct_geom *g, const char *who) {
 }
 
 void Workspace::free_buffers() {
-  DeviceBuffer *bufs[] = {&vol_pad, &proj_pad, &red, &filt_tmp, &ssim_ws, &bp_rects};
+  DeviceBuffer *bufs[] = {&vol_pad, &vol_cells, &proj_pad, &red, &filt_tmp, &ssim_ws, &bp_rects};
   for (auto *b : bufs) {
     if (b->ptr) (void)hipFree(b->ptr);
     b->ptr = nullptr;
@@ -270,7 +270,7 @@ const char *cbct_last_error(cbct_ctx ctx) {
 size_t cbct_workspace_bytes(cbct_ctx ctx) {
   if (!ctx) return 0;
   const Workspace &w = *ctx->ws;
-  return w.vol_pad.bytes + w.proj_pad.bytes + w.red.bytes + w.filt_tmp.bytes + w.ssim_ws.bytes +
+  return w.vol_pad.bytes + w.vol_cells.bytes + w.proj_pad.bytes + w.red.bytes + w.filt_tmp.bytes + w.ssim_ws.bytes +
          w.bp_rects.bytes;
 }
 

@@ -62,6 +62,7 @@ struct FPParams {
   float cx, cy, cz;           // clamp limits in padded texel space (= n_axis + 1)
   unsigned vg;                // column engine: views per launch group (see col_block)
   unsigned lds_stp;           // column engine: floats of LDS before the parked step lengths
+  int split;                  // column engine: rays not shared are k_fp_clip's
 };
 
 template <typename T>
@@ -416,6 +417,27 @@ __device__ __forceinline__ float2 zpair<unsigned short>(__amdgpu_buffer_rsrc_t r
   return make_float2(__uint_as_float(w << 16), __uint_as_float(w & 0xffff0000u));
 }
 
+// Elements e and e + 1 (z and z + 1) of k_pack_cells' copy: the voxel and its
+// neighbours at x + 1, y + 1 and both.
+template <typename T>
+__device__ __forceinline__ void cell_pair(__amdgpu_buffer_rsrc_t r, unsigned e, float4 &lo, float4 &hi);
+template <>
+__device__ __forceinline__ void cell_pair<float>(__amdgpu_buffer_rsrc_t r, unsigned e, float4 &lo, float4 &hi) {
+  const auto a = __builtin_amdgcn_raw_buffer_load_b128(r, (int)(e * 16u), 0, 0);
+  const auto b = __builtin_amdgcn_raw_buffer_load_b128(r, (int)(e * 16u + 16u), 0, 0);
+  lo = make_float4(__uint_as_float(a[0]), __uint_as_float(a[1]), __uint_as_float(a[2]), __uint_as_float(a[3]));
+  hi = make_float4(__uint_as_float(b[0]), __uint_as_float(b[1]), __uint_as_float(b[2]), __uint_as_float(b[3]));
+}
+template <>
+__device__ __forceinline__ void cell_pair<unsigned short>(__amdgpu_buffer_rsrc_t r, unsigned e, float4 &lo,
+                                                          float4 &hi) {
+  const auto v = __builtin_amdgcn_raw_buffer_load_b128(r, (int)(e * 8u), 0, 0);
+  auto low = [](unsigned w) { return __uint_as_float(w << 16); };
+  auto high = [](unsigned w) { return __uint_as_float(w & 0xffff0000u); };
+  lo = make_float4(low(v[0]), high(v[0]), low(v[1]), high(v[1]));
+  hi = make_float4(low(v[2]), high(v[2]), low(v[3]), high(v[3]));
+}
+
 // The sum over its n samples of each lane's ray R (lanes with mine unset: 0),
 // for 64 adjacent rows of one detector column whose x/y positions are their
 // own (rays that leave through the volume's top or bottom).  One ray per lane
@@ -427,13 +449,15 @@ __device__ __forceinline__ float2 zpair<unsigned short>(__amdgpu_buffer_rsrc_t r
 // engine's (the same bits).  The texture address unit binds it: it takes four
 // lanes per clock when they hit one line, else one lane per line, so lanes run
 // along a ray (steps of a clipped ray stay within a voxel or two; 28 cache
-// accesses per load) and not across rays (40).  256 x 256 x 160 voxels, 90
-// views of 512 x 384, 30% of the rays clipped: 8.4 ms for the whole
-// projection, 40.8 with one ray per lane.
+// accesses per load) and not across rays (40).  CELLS: the copy of k_pack_cells,
+// whose elements hold the four (x, y) corners: half the loads.  256 x 256 x 160
+// voxels, 90 views of 512 x 384, 30% of the rays clipped: 8.4 ms for the whole
+// projection from the plain copy, 5.6 from the packed one (k_fp_clip), 40.8 with
+// one ray per lane.
 //   lds: 64 x 6 floats of ray parameters, 64 x FPG_ROW floats of samples
 constexpr int FPG_ROW = 12;   // 8 samples, 16-byte aligned rows off the same banks
 constexpr int FPG_LDS = 64 * 6 + 64 * FPG_ROW;
-template <typename T>
+template <typename T, bool CELLS>
 __device__ __forceinline__ float fp_gather(const FPParams &P, const RaySetup &R, const bool mine,
                                            const T *__restrict__ vt, unsigned vt_bytes, int lane,
                                            float *lds) {
@@ -465,12 +489,22 @@ __device__ __forceinline__ float fp_gather(const FPParams &P, const RaySetup &R,
       const float ax = __builtin_amdgcn_fractf(sx), ay = __builtin_amdgcn_fractf(sy);
       const float az = __builtin_amdgcn_fractf(sz);
       const unsigned e = ((unsigned)(int)sy * P.px + (unsigned)(int)sx) * P.pz + (unsigned)(int)sz;
-      const float2 v00 = zpair<T>(rsrc, e, 0), v10 = zpair<T>(rsrc, e, so_x);
-      const float2 v01 = zpair<T>(rsrc, e, so_y), v11 = zpair<T>(rsrc, e, so_xy);
-      const float c00 = fmaf(ax, v10.x - v00.x, v00.x);
-      const float c10 = fmaf(ax, v11.x - v01.x, v01.x);
-      const float c01 = fmaf(ax, v10.y - v00.y, v00.y);
-      const float c11 = fmaf(ax, v11.y - v01.y, v01.y);
+      float c00, c10, c01, c11;   // x-lerped (y, z) corners
+      if constexpr (CELLS) {
+        float4 lo, hi;   // (x, y) corners at z and z + 1
+        cell_pair<T>(rsrc, e, lo, hi);
+        c00 = fmaf(ax, lo.y - lo.x, lo.x);
+        c10 = fmaf(ax, lo.w - lo.z, lo.z);
+        c01 = fmaf(ax, hi.y - hi.x, hi.x);
+        c11 = fmaf(ax, hi.w - hi.z, hi.z);
+      } else {
+        const float2 v00 = zpair<T>(rsrc, e, 0), v10 = zpair<T>(rsrc, e, so_x);
+        const float2 v01 = zpair<T>(rsrc, e, so_y), v11 = zpair<T>(rsrc, e, so_xy);
+        c00 = fmaf(ax, v10.x - v00.x, v00.x);
+        c10 = fmaf(ax, v11.x - v01.x, v01.x);
+        c01 = fmaf(ax, v10.y - v00.y, v00.y);
+        c11 = fmaf(ax, v11.y - v01.y, v01.y);
+      }
       const float c0 = fmaf(ay, c10 - c00, c00);
       const float c1 = fmaf(ay, c11 - c01, c01);
       smp[(8 * o + lr) * FPG_ROW + ls] = fmaf(az, c1 - c0, c0);
@@ -592,21 +626,9 @@ __device__ __forceinline__ void fp_col_body(const FPParams &P, const ViewD *__re
   qzl = of_row(qz, gjmin);
   pzh = of_row(pz, gjmax);
   qzh = of_row(qz, gjmax);
-  if (SSTEP && gjmax >= 0) {
-    // Every shared ray's z texel coordinate lies between the first and last
-    // shared rays' (monotone in the row) and, being linear in the step,
-    // between its values at the first and last step.  If all four are inside
-    // [0, nz+1] the per-ray z clamp is the identity and is dropped; otherwise
-    // the whole column takes the per-ray path.
-    const float ml = (float)(P.n - 1);
-    const float e1 = fmaf(ml, qzl, pzl), e3 = fmaf(ml, qzh, pzh);
-    const bool z_ok = fminf(fminf(pzl, e1), fminf(pzh, e3)) >= 0.0f &&
-                      fmaxf(fmaxf(pzl, e1), fmaxf(pzh, e3)) <= P.cz;
-    if (!z_ok) {
-      shared_mask = 0;
-      gjmax = -1;
-    }
-  }
+  // Shared rays leave through the x and y faces, so their z texel coordinates
+  // stay in [0.5, nz + 0.5] up to rounding (under 1e-3: nz <= 4096): the
+  // per-ray clamp to [0, nz + 1] is the identity and is dropped (SSTEP).
 
   if (SSTEP && gjmax >= 0) {
 #pragma unroll
@@ -868,7 +890,7 @@ __device__ __forceinline__ void fp_col_body(const FPParams &P, const ViewD *__re
   // The FP64 column setup is evaluated again (through an opaque copy of the
   // column index), which keeps its 20 registers out of the loops above.
   const unsigned todo = valid_mask & ~shared_mask;
-  if (__builtin_amdgcn_ballot_w64(todo != 0)) {
+  if (!P.split && __builtin_amdgcn_ballot_w64(todo != 0)) {
     int iw = __builtin_amdgcn_readfirstlane(i);
     asm volatile("" : "+s"(iw));
     const ViewD vw = views[k];
@@ -878,14 +900,14 @@ __device__ __forceinline__ void fp_col_body(const FPParams &P, const ViewD *__re
       const bool mine = (todo >> r) & 1u;
       if (__builtin_amdgcn_ballot_w64(mine) == 0) continue;
       const RaySetup R = ray_finish(P, vw, C, row0 + r * 64 + lane);
-      const float a = fp_gather<T>(P, R, mine, vt, vt_bytes, lane, zl);
+      const float a = fp_gather<T, false>(P, R, mine, vt, vt_bytes, lane, zl);
       if (mine) stp[64 * r] = a * R.step;
     }
   }
 
 #pragma unroll
   for (int r = 0; r < RPL; ++r) {
-    if (!(valid_mask & (1u << r))) continue;
+    if (!((P.split ? shared_mask : valid_mask) & (1u << r))) continue;
     const int j = row0 + r * 64 + lane;
     const size_t idx = (size_t)i + (size_t)P.nu * ((size_t)j + (size_t)P.nv * k);
     const float v = stp[64 * r];
@@ -913,6 +935,34 @@ k_fp_colc(FPParams P, const ViewD *__restrict__ views, const T *__restrict__ vt,
           float *__restrict__ proj, int accumulate, unsigned ngroups, unsigned nblocks,
           unsigned vt_bytes) {
   fp_col_body<T, RPL, true, 2, ZC, D>(P, views, vt, proj, accumulate, ngroups, nblocks, vt_bytes);
+}
+
+// The rays that the column kernels with P.split leave out (those not shared),
+// from the packed copy: one wave per 64 rows of a detector column.  Used where
+// many rays are clipped (clip_split).
+template <typename T>
+__global__ void __launch_bounds__(64) k_fp_clip(FPParams P, const ViewD *__restrict__ views,
+                                                const T *__restrict__ cells, float *__restrict__ proj,
+                                                int accumulate, unsigned nslots, unsigned nblocks,
+                                                unsigned cell_bytes) {
+  __shared__ __align__(16) float lds[FPG_LDS];
+  int i, slot, k;
+  col_block(P, xcd_remap(blockIdx.x, nblocks), nslots, nblocks, i, slot, k);
+  const int lane = threadIdx.x, j = slot * 64 + lane;
+  const ViewD vw = views[k];
+  const ColSetup C = col_setup(P, vw, i);
+  const double a1c = fmax(C.lo, 0.0), a2c = fmin(C.hi, 1.0);
+  const double t = fabs(P.lz * 0.5 / row_height(P, vw, j));
+  const bool shared = a2c - a1c >= 0.0 && fmax(fmax(C.lo, -t), 0.0) == a1c && fmin(fmin(C.hi, t), 1.0) == a2c;
+  const bool mine = j < P.nv && !shared;
+  if (__builtin_amdgcn_ballot_w64(mine) == 0) return;
+  const RaySetup R = ray_finish(P, vw, C, j);
+  const float a = fp_gather<T, true>(P, R, mine, cells, cell_bytes, lane, lds);
+  if (mine) {
+    const size_t idx = (size_t)i + (size_t)P.nu * ((size_t)j + (size_t)P.nv * k);
+    const float v = a * R.step;
+    proj[idx] = accumulate ? proj[idx] + v : v;
+  }
 }
 
 // ------------------------------------------------------------ layouts
@@ -973,6 +1023,27 @@ __global__ void __launch_bounds__(256) k_pad_transpose(const TI *__restrict__ vo
     const int xp = x0 + r, zp = z0 + tx;
     if (xp < (int)px && zp < (int)pz)
       out[(size_t)zp + (size_t)pz * ((size_t)xp + (size_t)px * yp)] = tile[tx][r];
+  }
+}
+
+// Packed copy for k_fp_clip: element e of the z-fastest copy (px columns of pz
+// per y) with its neighbours at x + 1, y + 1 and both, for x <= px - 2, y <= py
+// - 2 (the rest is never read).  Four z per thread and 16-byte loads.
+template <typename T>
+__global__ void __launch_bounds__(256) k_pack_cells(const T *__restrict__ vt, T *__restrict__ out, unsigned pz,
+                                                    unsigned px, unsigned py) {
+  const unsigned n4 = pz / 4 * px * (py - 1);   // pz is a multiple of 16
+  const size_t pzx = (size_t)pz * px;
+  struct __align__(4 * sizeof(T)) V4 {
+    T v[4];
+  };
+  for (unsigned t = blockIdx.x * 256 + threadIdx.x; t < n4; t += gridDim.x * 256) {
+    const size_t e = (size_t)t * 4;
+    if (t / (pz / 4) % px == px - 1) continue;
+    const V4 a = *reinterpret_cast<const V4 *>(vt + e), b = *reinterpret_cast<const V4 *>(vt + e + pz);
+    const V4 c = *reinterpret_cast<const V4 *>(vt + e + pzx), d = *reinterpret_cast<const V4 *>(vt + e + pzx + pz);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) *reinterpret_cast<V4 *>(out + 4 * (e + i)) = V4{{a.v[i], b.v[i], c.v[i], d.v[i]}};
   }
 }
 
@@ -1037,6 +1108,8 @@ int make_params(cbct_ctx ctx, const cbct_geom *g, float spp, FPParams &P) {
   P.cy = (float)(g->ny + 1);
   P.cz = (float)(g->nz + 1);
   P.vg = (unsigned)ctx->fp_view_group;
+  P.lds_stp = 0;
+  P.split = 0;
   return CBCT_OK;
 }
 
@@ -1262,6 +1335,25 @@ size_t fp_working_bytes(cbct_ctx ctx, const cbct_geom *g, const FPParams &P, int
   return ((size_t)P.pzx * padded_dim(g->ny) + 1024) * esz;
 }
 
+// Whether the rays that leave through the top or bottom go to k_fp_clip: when
+// their samples (those of the rows that reach past the volume's height at its
+// far side, an upper bound) outweigh building the packed copy.  The copy costs
+// 20 bytes of traffic per voxel (4.4 ps), the packed loads save about 1.6 ps a
+// sample.  The copy must stay within a buffer's 4 GB.
+bool clip_split(cbct_ctx ctx, const cbct_geom *g, const FPParams &P, int view0, int nviews, size_t esz) {
+  if ((size_t)P.pzx * padded_dim(g->ny) * 4 * esz >= (1ull << 32) - 64) return false;
+  const double R = 0.5 * std::sqrt((double)g->lx * g->lx + (double)g->ly * g->ly);
+  const double vmax = 0.5 * g->lz * g->sdd / ((double)g->sad + R);   // heights up to here are never clipped
+  const double pitch = (double)g->fov_v / g->nv;
+  double rows = 0.0;
+  for (int k = 0; k < nviews; ++k) {
+    const double off = ctx->offsets[2 * (size_t)(view0 + k) + 1];
+    rows += std::max(0.0, 0.5 * g->fov_v + off - vmax) / pitch + std::max(0.0, 0.5 * g->fov_v - off - vmax) / pitch;
+  }
+  const double samples = rows * g->nu * P.n, nvox = (double)g->nx * g->ny * g->nz;
+  return samples > 3.6 * nvox;
+}
+
 // TI: the caller's volume type; T: the padded working copy's type.  The
 // working copy goes to the context's workspace, or to `ext` when given (the
 // caller has checked it holds fp_working_bytes).
@@ -1306,8 +1398,29 @@ int run_fp(cbct_ctx ctx, const cbct_geom *g, const FPParams &P, int view0, int n
   CBCT_LAUNCH_CHECK(ctx, "k_pad_transpose");
   FPParams Q = P;
   if (choice.vg > 0) Q.vg = (unsigned)choice.vg;
+  // without memory for the packed copy the column kernels take every ray
+  Q.split = !ext && clip_split(ctx, g, P, view0, nviews, esz) &&
+            cbct_reserve(ctx, ctx->ws->vol_cells, 4 * npad * esz) == CBCT_OK;
+  const unsigned nslots = ceil_div(P.nv, 64);
+  const unsigned cell_bytes = (unsigned)(4 * npad * esz);
+  T *cells = static_cast<T *>(ctx->ws->vol_cells.ptr);
+  if (Q.split) {
+    hipLaunchKernelGGL(k_pack_cells<T>, dim3(std::min(ceil_div(npad / 4, 256), 65536u)), dim3(256), 0, s, vt, cells,
+                       P.pz, P.px, (unsigned)py);
+    CBCT_LAUNCH_CHECK(ctx, "k_pack_cells");
+  }
   cbct_prof_mark(ctx, PROF_FP, 0, s);
   dispatch_col<T>(Q, choice, s, views, vt, proj, accumulate, nviews, (unsigned)vt_bytes);
+  if (Q.split) {
+    // at most 2^32 - 1 work-items per launch, as launch_col
+    const size_t per_view = (size_t)P.nu * nslots;
+    const int max_views = (int)std::max<size_t>(1, std::min<size_t>(nviews, ((1ull << 32) - 1) / 64 / per_view));
+    for (int v0 = 0; v0 < nviews; v0 += max_views) {
+      const unsigned nblocks = (unsigned)(per_view * (size_t)std::min(max_views, nviews - v0));
+      hipLaunchKernelGGL(k_fp_clip<T>, dim3(nblocks), dim3(64), 0, s, Q, views + v0, cells,
+                         proj + (size_t)v0 * P.nu * P.nv, accumulate, nslots, nblocks, cell_bytes);
+    }
+  }
   cbct_prof_mark(ctx, PROF_FP, 1, s);
   CBCT_LAUNCH_CHECK(ctx, "k_fp_col");
   return CBCT_OK;

@@ -23,7 +23,9 @@
 // is idle; when the head of the queue does not fit, idle lanes free theirs.
 #include <hip/hip_runtime_api.h>
 
+#include <algorithm>
 #include <chrono>
+#include <cmath>
 #include <condition_variable>
 #include <cstring>
 #include <deque>
@@ -74,6 +76,8 @@ double ms(Clock::time_point a, Clock::time_point b) {
 //  FDK: the image and the padded volume copy (2.3 volumes); the projections,
 //    the filtered projections, A f, the filter staging and the padded copy of
 //    all views (up to 4x as quad texels): 8 sinograms.
+//  Both: where rays leave through the volume's top or bottom, the forward
+//    projector's packed copy (4 padded volumes).
 size_t footprint_bytes(const gtt_request &r) {
   const size_t nvox = (size_t)r.geom.nx * r.geom.ny * r.geom.nz;
   const size_t nproj = (size_t)(r.geom.nu + 3) * (r.geom.nv + 3) * (size_t)r.nviews;
@@ -81,10 +85,18 @@ size_t footprint_bytes(const gtt_request &r) {
   // the LDS-staged backprojector's rectangle table: 8 bytes per 16 x 16 x 8
   // (or x 16) voxel block and view of one backprojection call
   const size_t blocks = (size_t)((r.geom.nx + 15) / 16) * ((r.geom.ny + 15) / 16) * ((r.geom.nz + 7) / 8);
-  if (r.kind == GTT_REQ_FDK) return 4 * (nvox * 23 / 10 + 8 * nproj) + 8 * blocks * (size_t)r.nviews + slack;
+  double vtop = 0.5 * r.geom.fov_v;   // largest detector height, offsets included
+  if (r.offsets)
+    for (int k = 0; k < r.nviews; ++k)
+      vtop = std::max(vtop, 0.5 * r.geom.fov_v + std::fabs((double)r.offsets[2 * k + 1]));
+  const double R = 0.5 * std::hypot((double)r.geom.lx, (double)r.geom.ly);
+  const bool clipped = vtop * ((double)r.geom.sad + R) > 0.5 * r.geom.lz * r.geom.sdd;
+  const size_t packed = clipped ? 4 * (nvox * 52 / 10) : 0;
+  if (r.kind == GTT_REQ_FDK)
+    return 4 * (nvox * 23 / 10 + 8 * nproj) + 8 * blocks * (size_t)r.nviews + packed + slack;
   const size_t S = r.subsets > 0 ? (size_t)r.subsets : 1;
   return 4 * (nvox * (10 * S + 33) / 10 + 4 * nproj + 4 * ((nproj + S - 1) / S)) +
-         8 * blocks * (((size_t)r.nviews + S - 1) / S) + slack;
+         8 * blocks * (((size_t)r.nviews + S - 1) / S) + packed + slack;
 }
 
 // The request's storage type is the lane's default while its operators are

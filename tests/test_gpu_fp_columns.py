@@ -59,6 +59,12 @@ def test_clipped_rays(ctx, case, dtype):
     ctx.set_views(angles, offsets)
     a, b = project(ctx, g, v, 5, 0), project(ctx, g, v, 5, 1)
     assert torch.equal(a, b)
+    # without memory of its own the call takes them from the plain copy
+    c = torch.zeros_like(a)
+    ctx.fp_noalloc(g, v, c)
+    assert torch.equal(a, c)
+    ctx.fp(g, v, c, accumulate=True)
+    assert torch.equal(a + a, c)
     ref = O.fp(to_oracle(g), angles, offsets, v.double().cpu().numpy())
     assert rel_l2(b.cpu().numpy(), ref) <= TOL
 
