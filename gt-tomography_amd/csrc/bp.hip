@@ -36,8 +36,9 @@ struct BPParams {
   unsigned pview;      // padded elements per view
   unsigned pnu2;       // pair copy: row length (pnu rounded up to 4)
   unsigned pview2;     // pair copy: dwords per view
-  unsigned bpp_rowb;   // LDS row of the pair kernel in bytes (a parameter, so
+  unsigned bpp_rowb;   // LDS row of the staged kernel in bytes (a parameter, so
                        // the compiler keeps iv * row + col one 24-bit mad)
+  int bpp_rw, bpp_cap; // its LDS row and buffer in elements
 };
 
 template <typename T>
@@ -177,14 +178,26 @@ __global__ void __launch_bounds__(BP_TX *BP_TY) k_bp(BPParams P, const ViewF *__
 // copies, k_pad_staged): element (a, b) holds the taps (a, b) and (a+1, b), so
 // the four taps of a voxel-view are two elements one LDS row apart, one
 // ds_read2_b32; plain FP32 (k_pad_staged): the four taps are two adjacent
-// pairs of elements one row apart, two ds_read2_b32.  LDS rows are BPP_RW =
-// 68 elements (adjacent rows 4 banks apart); a buffer holds BPP_CAP
-// elements, a multiple of one 64-lane copy (256), so whole copies never write
-// past it.  Views whose rectangle does not fit read the copy directly.  Same
-// arithmetic, same bits as k_bp.
-constexpr int BPP_RW = 68;
-constexpr int BPP_CAP = 13 * 256;   // 48 rows of 68 elements, rounded up to whole copies
-constexpr int BPP_CHUNKS = BPP_CAP / 256;
+// pairs of elements one row apart, two ds_read2_b32.  Views whose rectangle
+// does not fit read the copy directly.  Same arithmetic, same bits as k_bp.
+//
+// LDS rows are RW elements; a buffer holds 48 of them, rounded up to whole
+// 64-lane copies (256 elements), so whole copies never write past it.  A wave's
+// taps at one z spread over 2-3 rows and up to 22 columns, so the rows' distance
+// in banks (RW mod 64) decides the bank conflicts, which with the FP32 kernel's
+// two reads per update are a quarter of its time at RW = 68; a narrow row also
+// copies less and lets a seventh block in.  512^3, 720 views, FP32 / FP32 with
+// FDK weight / BF16: RW 52 30.1 / 31.0 / 28.9 ms, 56 30.2 / 31.5 / 28.6, 60 32.6 /
+// 33.5 / 29.0, 68 33.7 / 34.6 / 29.5, 76 31.9 / 32.3 / 30.3.
+constexpr int BPP_NARROW = 52;                                  // where the rectangles fit
+constexpr int bpp_wide(bool pairs) { return pairs ? 68 : 76; }  // else
+constexpr int bpp_cap(int rw) { return (48 * rw + 255) / 256 * 256; }
+// Waves per SIMD of the FP32 kernels, whose earlier LDS reads take registers:
+// 512^3, 720 views, narrow rows, without / with the FDK weight: six 30.1 / 31.3
+// ms, seven 31.4 / 31.0, eight 31.6 / 31.1.
+constexpr int bpp_waves(bool pairs, bool fbp, int rw) {
+  return pairs ? 6 : rw != BPP_NARROW ? 5 : fbp ? 7 : 6;
+}
 
 // The rectangle of block L (x fastest, z slowest, as k_bpp) at view k, as
 // entry L * nviews + k: (u0 | v0 << 16, H | inner << 8), 0 when it does not
@@ -232,21 +245,26 @@ __global__ void __launch_bounds__(256) k_bpp_rects(BPParams P, const ViewF *__re
   const int u0 = max(ulo - 1, 0) & ~3, v0 = max(vlo - 1, 0);
   const int W = min(uhi + 2, (int)P.pnu2 - 1) - u0 + 1;
   const int H = min(vhi + 2, (int)P.pnv - 1) - v0 + 1;
-  const bool staged = W <= BPP_RW && H * BPP_RW <= BPP_CAP;
+  const bool staged = W <= P.bpp_rw && H * P.bpp_rw <= P.bpp_cap;
   // bit 8: every voxel's row coordinate lies inside [0, nv + 1] (half a
   // texel of margin), so its clamp is the identity and is skipped
   const unsigned inner = rlo >= 0.5f && rhi <= P.clv - 0.5f ? 0x100u : 0u;
   rects[t] = make_uint2((unsigned)u0 | ((unsigned)v0 << 16), staged ? (unsigned)H | inner : 0u);
 }
 
-template <bool PAIRS, bool FBP, int KZ>
-__global__ void __launch_bounds__(BP_TX *BP_TY) k_bpp(BPParams P, const ViewF *__restrict__ views,
-                                                      const unsigned *__restrict__ copy,
-                                                      const uint2 *__restrict__ rects,
-                                                      float *__restrict__ vol, int accumulate,
-                                                      unsigned gx, unsigned gy) {
+// 16 bytes per lane straight into LDS (dst: the wave's first lane's place).  Not
+// in the kernel template: there the host pass drops the kernel's stub.
+__device__ __forceinline__ void copy_to_lds(__amdgpu_buffer_rsrc_t r, unsigned *dst, unsigned voff) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void *)dst, 16, voff, 0, 0, 0);
+}
+
+template <bool PAIRS, bool FBP, int KZ, int RW>
+__global__ void __launch_bounds__(BP_TX *BP_TY) __attribute__((amdgpu_waves_per_eu(bpp_waves(PAIRS, FBP, RW))))
+k_bpp(BPParams P, const ViewF *__restrict__ views, const unsigned *__restrict__ copy,
+      const uint2 *__restrict__ rects, float *__restrict__ vol, int accumulate, unsigned gx, unsigned gy) {
 #pragma clang fp contract(off)
-  __shared__ unsigned buf[2 * BPP_CAP];
+  constexpr int CAP = bpp_cap(RW), CHUNKS = CAP / 256;
+  __shared__ unsigned buf[2 * CAP];
   // linear tile id, x fastest, z slowest (consecutive tiles land on
   // different XCDs, so all XCDs work on one band of detector rows per view)
   const unsigned L = blockIdx.x;
@@ -267,12 +285,12 @@ __global__ void __launch_bounds__(BP_TX *BP_TY) k_bpp(BPParams P, const ViewF *_
   // byte offset, within a rectangle, of the 4 elements each lane copies for
   // this wave's copies (copy i = wv + 4 j covers LDS elements [256 i, 256 i +
   // 256)); rows past the rectangle land in the buffer's unused tail
-  unsigned loff[(BPP_CHUNKS + 3) / 4];
+  unsigned loff[(CHUNKS + 3) / 4];
 #pragma unroll
-  for (int j = 0; j < (BPP_CHUNKS + 3) / 4; ++j) {
+  for (int j = 0; j < (CHUNKS + 3) / 4; ++j) {
     const int p = (wv + 4 * j) * 256 + ln * 4;
-    const int r = p / BPP_RW;
-    loff[j] = (unsigned)(r * (int)P.pnu2 + (p - r * BPP_RW)) * 4u;
+    const int r = p / RW;
+    loff[j] = (unsigned)(r * (int)P.pnu2 + (p - r * RW)) * 4u;
   }
   auto issue = [&](int k, uint2 R, int base) {
     // the rectangle's origin goes into the descriptor, so the hardware range
@@ -281,13 +299,11 @@ __global__ void __launch_bounds__(BP_TX *BP_TY) k_bpp(BPParams P, const ViewF *_
     const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
         (void *)((const char *)(copy + (size_t)k * P.pview2) + org), (short)0, (int)(view_bytes - org),
         0x00020000);
-    const int n = ((int)(R.y & 0xffu) * BPP_RW + 255) >> 8;
+    const int n = ((int)(R.y & 0xffu) * RW + 255) >> 8;
 #pragma unroll
-    for (int j = 0; j < (BPP_CHUNKS + 3) / 4; ++j)
+    for (int j = 0; j < (CHUNKS + 3) / 4; ++j)
       if (wv + 4 * j < n)
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(
-            rs, (__attribute__((address_space(3))) void *)&buf[base + (wv + 4 * j) * 256], 16, loff[j], 0,
-            0, 0);
+        copy_to_lds(rs, &buf[base + (wv + 4 * j) * 256], loff[j]);
   };
   float acc[KZ];
 #pragma unroll
@@ -317,7 +333,7 @@ __global__ void __launch_bounds__(BP_TX *BP_TY) k_bpp(BPParams P, const ViewF *_
     // have, and nobody reads view k-1's buffer any more
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
-    if (k + 1 < P.nviews && nxt.y) issue(k + 1, nxt, ((k + 1) & 1) * BPP_CAP);
+    if (k + 1 < P.nviews && nxt.y) issue(k + 1, nxt, ((k + 1) & 1) * CAP);
     auto tap = [&](int t, float a, float b, float c, float d, float av) {
       const float r0 = fmaf(au, b - a, a);
       const float r1 = fmaf(au, d - c, c);
@@ -339,7 +355,7 @@ __global__ void __launch_bounds__(BP_TX *BP_TY) k_bpp(BPParams P, const ViewF *_
       // LDS byte address of element (iv, iu): iv * row + iu * 4 + s, with s
       // uniform (readfirstlane keeps the compiler from splitting the sum)
       const unsigned s = __builtin_amdgcn_readfirstlane(
-          (unsigned)(((k & 1) * BPP_CAP - (int)(cur.x & 0xffffu) - (int)(cur.x >> 16) * BPP_RW) * 4));
+          (unsigned)(((k & 1) * CAP - (int)(cur.x & 0xffffu) - (int)(cur.x >> 16) * RW) * 4));
       const unsigned colb = (unsigned)iu * 4u + s;
       const char *lds = (const char *)buf;
       auto ld = [&](unsigned o) { return *(const unsigned *)(lds + o); };
@@ -349,14 +365,14 @@ __global__ void __launch_bounds__(BP_TX *BP_TY) k_bpp(BPParams P, const ViewF *_
         for (int t = 0; t < KZ; ++t) {
           const float tv = fmaf((float)t, dtv, tv0);
           taps(t, __builtin_amdgcn_fractf(tv), ld, __umul24((unsigned)(int)tv, P.bpp_rowb) + colb,
-               BPP_RW * 4u);
+               RW * 4u);
         }
       } else {
 #pragma unroll
         for (int t = 0; t < KZ; ++t) {
           const float tv = __builtin_amdgcn_fmed3f(fmaf((float)t, dtv, tv0), 0.0f, P.clv);
           taps(t, __builtin_amdgcn_fractf(tv), ld, __umul24((unsigned)(int)tv, P.bpp_rowb) + colb,
-               BPP_RW * 4u);
+               RW * 4u);
         }
       }
     } else {
@@ -601,7 +617,6 @@ BPParams make_params(const cbct_geom *g, int nviews) {
   P.pview = (unsigned)(padded_dim(g->nu) * padded_dim(g->nv));
   P.pnu2 = (P.pnu + 3u) & ~3u;
   P.pview2 = P.pnu2 * P.pnv;
-  P.bpp_rowb = BPP_RW * 4;
   return P;
 }
 
@@ -617,13 +632,16 @@ inline int bp_kz(const cbct_ctx ctx, const cbct_geom *g) {
   return tiles16 < 1024 ? 8 : KZ;
 }
 
-// Whether the LDS-staged kernel should run: at least half of the blocks'
-// detector rectangles fit its LDS tile (staged block-views take about 0.7 of
-// the quad kernel's time; with a quarter staged the two were measured equal
-// at BF16), estimated on up to 8 evenly spaced views x a grid of up to 16 x
-// 16 block columns x every z-band, with one texel of slack on each side.
-// Cached per geometry, view range and z-depth until the view table changes.
-bool bpp_fits(cbct_ctx ctx, const cbct_geom *g, const BPParams &P, int view0, int nviews, int kz) {
+// Whether the LDS-staged kernel should run, and with which rows: 0 = no, 1 =
+// wide, 2 = narrow.  Staged when at least half of the blocks' detector
+// rectangles fit 68-element rows (staged block-views take about 0.7 of the quad
+// kernel's time; with a quarter staged the two were measured equal at BF16);
+// narrow when at least 0.9 of them fit those (200^3 / 430 columns: 0.82 fit,
+// narrow and wide equal; 291^3 / 667: 0.73 fit, narrow 0.344 ms, wide 0.320).
+// Estimated on up to 8 evenly spaced views x a grid of up to 16 x 16 block
+// columns x every z-band, with one texel of slack on each side.  Cached per
+// geometry, view range and z-depth until the view table changes.
+int bpp_fits(cbct_ctx ctx, const cbct_geom *g, const BPParams &P, int view0, int nviews, int kz) {
   std::vector<float> key = {(float)g->nx, (float)g->ny, (float)g->nz, g->lx, g->ly, g->lz,
                             (float)g->nu, (float)g->nv, g->fov_u, g->fov_v, g->sad, g->sdd,
                             (float)view0, (float)nviews, (float)kz};
@@ -633,7 +651,7 @@ bool bpp_fits(cbct_ctx ctx, const cbct_geom *g, const BPParams &P, int view0, in
   const int gzb = (int)ceil_div(g->nz, kz);
   const float dz = P.lz / P.nz;
   const int vstep = std::max(1, nviews / 8), sx = std::max(1, gx / 16), sy = std::max(1, gy / 16);
-  size_t total = 0, staged = 0;
+  size_t total = 0, staged = 0, narrow = 0;
   for (int k = view0; k < view0 + nviews; k += vstep) {
     const ViewF vw = ctx->views_h[k];
     for (int by = 0; by < gy; by += sy)
@@ -655,7 +673,7 @@ bool bpp_fits(cbct_ctx ctx, const cbct_geom *g, const BPParams &P, int view0, in
         total += gzb;
         const int u0 = std::max((int)std::floor(ulo) - 2, 0) & ~3;
         const int W = std::min((int)std::floor(uhi) + 3, (int)P.pnu2 - 1) - u0 + 1;
-        if (W > BPP_RW) continue;
+        if (W > 68) continue;
         for (int zb = 0; zb < gzb; ++zb) {
           // v is linear in pz * mag: extreme at the band's end slices and the
           // extreme magnifications
@@ -667,33 +685,42 @@ bool bpp_fits(cbct_ctx ctx, const cbct_geom *g, const BPParams &P, int view0, in
           const float vhi = std::min(std::max((phi - vw.off_v) * P.sv + P.cv, 0.0f), P.clv);
           const int v0 = std::max((int)std::floor(vlo) - 2, 0);
           const int H = std::min((int)std::floor(vhi) + 3, (int)P.pnv - 1) - v0 + 1;
-          staged += H * BPP_RW <= BPP_CAP;
+          staged += H * 68 <= bpp_cap(68);
+          narrow += W <= BPP_NARROW && H * BPP_NARROW <= bpp_cap(BPP_NARROW);
         }
       }
   }
-  const bool fits = staged * 2 >= total;
+  const int fits = staged * 2 < total ? 0 : narrow * 10 >= total * 9 ? 2 : 1;
   if (ctx->bpp_fit_cache.size() >= 256) ctx->bpp_fit_cache.clear();
   ctx->bpp_fit_cache.emplace_back(std::move(key), fits);
   return fits;
 }
 
-// Whether the call runs the LDS-staged kernel (engine 2 where it pays,
-// engine 3 always; rectangle origins are packed in 16 bits).
-bool use_staged(cbct_ctx ctx, const cbct_geom *g, const BPParams &P, int view0, int nviews, int kz) {
-  return ctx->bp_engine >= 2 && P.pnu2 < 65536 && P.pnv < 65536 &&
-         (ctx->bp_engine == 3 || bpp_fits(ctx, g, P, view0, nviews, kz));
+// Whether the call runs the LDS-staged kernel (engine 2 where it pays, engine 3
+// always; rectangle origins are packed in 16 bits), as bpp_fits.
+int use_staged(cbct_ctx ctx, const cbct_geom *g, const BPParams &P, int view0, int nviews, int kz) {
+  if (ctx->bp_engine < 2 || P.pnu2 >= 65536 || P.pnv >= 65536) return 0;
+  const int fits = bpp_fits(ctx, g, P, view0, nviews, kz);
+  return ctx->bp_engine == 3 ? std::max(fits, 1) : fits;
 }
 
-template <bool PAIRS, int Z>
+template <bool PAIRS, int Z, int RW>
 void launch_bpp(const BPParams &P, dim3 grid, hipStream_t s, const ViewF *views, const unsigned *cp,
                 const uint2 *rects, float *vol, int fbp, int acc) {
   const unsigned nblocks = grid.x * grid.y * grid.z;
   if (fbp)
-    hipLaunchKernelGGL((k_bpp<PAIRS, true, Z>), dim3(nblocks), dim3(BP_TX, BP_TY), 0, s, P, views, cp,
+    hipLaunchKernelGGL((k_bpp<PAIRS, true, Z, RW>), dim3(nblocks), dim3(BP_TX, BP_TY), 0, s, P, views, cp,
                        rects, vol, acc, grid.x, grid.y);
   else
-    hipLaunchKernelGGL((k_bpp<PAIRS, false, Z>), dim3(nblocks), dim3(BP_TX, BP_TY), 0, s, P, views, cp,
+    hipLaunchKernelGGL((k_bpp<PAIRS, false, Z, RW>), dim3(nblocks), dim3(BP_TX, BP_TY), 0, s, P, views, cp,
                        rects, vol, acc, grid.x, grid.y);
+}
+
+template <bool PAIRS, int Z>
+void launch_bpp_rows(const BPParams &P, int rows, dim3 grid, hipStream_t s, const ViewF *views,
+                     const unsigned *cp, const uint2 *rects, float *vol, int fbp, int acc) {
+  if (rows == 2) launch_bpp<PAIRS, Z, BPP_NARROW>(P, grid, s, views, cp, rects, vol, fbp, acc);
+  else launch_bpp<PAIRS, Z, bpp_wide(PAIRS)>(P, grid, s, views, cp, rects, vol, fbp, acc);
 }
 
 template <typename T, bool QUAD, int Z>
@@ -718,11 +745,15 @@ void launch_bp(const BPParams &P, dim3 grid, int kz, hipStream_t s, const ViewF 
 // Padded copy in the selected layout (and storage type), then the kernel.
 // TI: the caller's projection type; T: the copy's.
 template <typename TI, typename T>
-int run_bp(cbct_ctx ctx, const cbct_geom *g, const BPParams &P, dim3 grid, int kz, int view0,
+int run_bp(cbct_ctx ctx, const cbct_geom *g, BPParams P, dim3 grid, int kz, int view0,
            int nviews, const TI *proj, float *vol, int fbp, int accumulate, hipStream_t s) {
   // the LDS-staged kernel on a pair copy for BF16 working copies, a plain
   // one for FP32, after the pass that computes its rectangles
-  if (use_staged(ctx, g, P, view0, nviews, kz)) {
+  if (const int rows = use_staged(ctx, g, P, view0, nviews, kz)) {
+    constexpr bool PAIRS = sizeof(T) == 2;
+    P.bpp_rw = rows == 2 ? BPP_NARROW : bpp_wide(PAIRS);
+    P.bpp_cap = bpp_cap(P.bpp_rw);
+    P.bpp_rowb = (unsigned)P.bpp_rw * 4u;
     int rc2 = cbct_reserve(ctx, ctx->ws->proj_pad, (size_t)P.pview2 * nviews * 4);
     if (rc2) return rc2;
     const size_t nblocks = (size_t)grid.x * grid.y * grid.z;
@@ -748,8 +779,10 @@ int run_bp(cbct_ctx ctx, const cbct_geom *g, const BPParams &P, dim3 grid, int k
                          grid.x, grid.y, (unsigned)nblocks);
     CBCT_LAUNCH_CHECK(ctx, "k_bpp_rects");
     cbct_prof_mark(ctx, PROF_BP, 0, s);
-    if (kz == 8) launch_bpp<sizeof(T) == 2, 8>(P, grid, s, vf, cp, rects, vol, fbp, accumulate);
-    else launch_bpp<sizeof(T) == 2, KZ>(P, grid, s, vf, cp, rects, vol, fbp, accumulate);
+    if (kz == 8)
+      launch_bpp_rows<PAIRS, 8>(P, rows, grid, s, vf, cp, rects, vol, fbp, accumulate);
+    else
+      launch_bpp_rows<PAIRS, KZ>(P, rows, grid, s, vf, cp, rects, vol, fbp, accumulate);
     cbct_prof_mark(ctx, PROF_BP, 1, s);
     CBCT_LAUNCH_CHECK(ctx, "k_bpp");
     return CBCT_OK;

@@ -66,10 +66,10 @@ struct cbct_ctx_s {
   int filter_engine = 2;
   int fp_engine = 1;             // 1: detector-column sharing, 0: one thread per ray
   int bp_engine = 2;             // 2: LDS-staged, 3: LDS-staged forced (BF16), 1: quad, 0: plain
-  // backprojector: whether the LDS tile of the BF16 pair kernel holds the
-  // blocks' detector rectangles, per (geometry, views, z-depth); cleared
-  // with the view table
-  std::vector<std::pair<std::vector<float>, bool>> bpp_fit_cache;
+  // backprojector: whether (and with which rows) the staged kernel's LDS tile
+  // holds the blocks' detector rectangles, per (geometry, views, z-depth);
+  // cleared with the view table
+  std::vector<std::pair<std::vector<float>, int>> bpp_fit_cache;
   int bp_kz = 0;                 // z-voxels per BP thread: 0 = chosen by size, else 8 or 16
   int fp_max_rpl = 0;            // column engine: most detector rows per lane; 0 = unset (8; engine 1: 12)
   int fp_view_group = 6;         // column engine: adjacent views launched together per column
