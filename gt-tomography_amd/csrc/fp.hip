@@ -1151,10 +1151,10 @@ struct FPChoice {
   int rpl;      // rows per lane
   int zc = 0;
   int vg = 0;   // views per launch group; 0 = the context's setting
-  bool deep = false;   // cached variant with the lines of four steps in flight
 };
-// Deep variants: windows of 64 and 128 z, up to 4 rows per lane, for launches
-// of fewer waves than hide each other's latencies (8 per SIMD).  64^3, 9 views
+// Deep variants (the lines of four steps in flight): windows of 64 and 128 z, up
+// to 4 rows per lane, for launches of fewer waves than hide each other's
+// latencies (8 per SIMD); a property of each launch, also of a tuned choice.  64^3, 9 views
 // (864 waves) 40 -> 31 us with the padded copy, 96^3, 10 views (1500) 61 -> 51,
 // 128^3, 24 views (6144) 136 -> 125; from 12288 waves on they cost 2-9%, and
 // with wider windows they gain nothing.
@@ -1167,8 +1167,10 @@ void launch_col_w(const FPParams &P, const FPChoice &c, hipStream_t s, const Vie
   if (c.variant == 1) return launch_col<T, RPL, false, 1, 0>(P, s, views, vt, proj, acc, nviews, vt_bytes);
   if (c.variant == 2) return launch_col<T, RPL, true, 2, 0>(P, s, views, vt, proj, acc, nviews, vt_bytes);
   if constexpr (RPL <= FP_DEEP_RPL) {
-    if (c.deep && c.zc == 1) return launch_col<T, RPL, true, 2, 1, 4>(P, s, views, vt, proj, acc, nviews, vt_bytes);
-    if (c.deep && c.zc == 2) return launch_col<T, RPL, true, 2, 2, 4>(P, s, views, vt, proj, acc, nviews, vt_bytes);
+    const size_t groups = (P.nv + 64 * RPL - 1) / (64 * RPL);
+    const bool deep = c.zc <= FP_DEEP_ZC && groups * P.nu * nviews < FP_DEEP_WAVES;
+    if (deep && c.zc == 1) return launch_col<T, RPL, true, 2, 1, 4>(P, s, views, vt, proj, acc, nviews, vt_bytes);
+    if (deep && c.zc == 2) return launch_col<T, RPL, true, 2, 2, 4>(P, s, views, vt, proj, acc, nviews, vt_bytes);
   }
   switch (c.zc) {
     case 1: launch_col<T, RPL, true, 2, 1>(P, s, views, vt, proj, acc, nviews, vt_bytes); break;
@@ -1272,8 +1274,6 @@ FPChoice default_variant(cbct_ctx ctx, const cbct_geom *g, const FPParams &P, in
     if (zc <= FP_ZC_MAX && cost < best_cost) {
       best_cost = cost;
       best = {3, rpl, zc};
-      best.deep = zc <= FP_DEEP_ZC && rpl <= FP_DEEP_RPL &&
-                  (size_t)groups * P.nu * nviews < FP_DEEP_WAVES;
     }
   }
   return best;
