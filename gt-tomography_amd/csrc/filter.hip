@@ -703,7 +703,7 @@ __device__ __forceinline__ void fft_pass(cf (&a)[P], const cf (&w)[NT]) {
 }
 
 // LDS padding of the exchange after pass NS (positions p < N, padded below
-// N + N/8): the pass's writes and the next pass's reads both fall on
+// N + N/P): the pass's writes and the next pass's reads both fall on
 // distinct banks for every 32 lanes (64 banks of 4 bytes, 8-byte points).
 // After the first pass (writes P apart): p + p/32; after the second (groups
 // of P consecutive, P^2 apart): p + P (p / P^2); later passes write
@@ -778,16 +778,24 @@ struct FftShape {
   static constexpr int G = N >= 2048 ? 1 : 2048 / N;   // row pairs per workgroup
   static constexpr int T = G * N / P;                  // threads
   static constexpr int RL = N >> (LP * ((LOG2N - 1) / LP));   // radix of the last pass
-  static constexpr int PN = N + N / 8;                 // padded length of one pair's buffer
+  static constexpr int PN = N + N / P;                 // padded length of one pair's buffer
 };
 
 // Persistent: workgroup b takes pair groups b, b + gridDim.x, ...; the next
 // group's rows (and cosine weights) are loaded while this one transforms.
-// PARKER: the short-scan weights, in an instantiation of their own (their
-// range reductions would otherwise set the common kernel's register count).
+// PARKER: the short-scan weights.  They depend on the column and the view only,
+// and forming them (four sines with their range reductions and an arc tangent
+// per pixel) took three times the transforms' time, at one wave per SIMD for its
+// registers.  So a workgroup takes a contiguous run of groups, a group's rows
+// are of one view (`plane` rows each: a last group may have fewer), and a
+// thread forms the weights of its columns when the view changes, in a loop,
+// and keeps them in LDS slots of its own (no barrier): 1024 x 768, 180 views
+// 1317 -> 415 us, 512 x 383 355 -> 124, 200 x 150, 150 views 79 -> 42.  Contiguous
+// runs cost the plain instantiation 3% (1024 workgroups then read as many
+// places of memory at once), also when they share their cosine weights.
 template <int LOG2N, bool PARKER>
 __global__ void __launch_bounds__(FftShape<LOG2N>::T) k_ramp_fft(
-    const float *in, float *out, size_t nrows, int nu, const cf *__restrict__ tw,
+    const float *in, float *out, size_t nrows, size_t plane, int nu, const cf *__restrict__ tw,
     const float *__restrict__ cs, const float *__restrict__ cosw, int nv,
     const float *__restrict__ angles, float delta, float tan_delta) {
   using S = FftShape<LOG2N>;
@@ -798,8 +806,14 @@ __global__ void __launch_bounds__(FftShape<LOG2N>::T) k_ramp_fft(
   __shared__ cf buf[2][G * PN];
   __shared__ double part[2][NW];
   __shared__ float partf[2][NW];
+  __shared__ float pkw[PARKER ? H : 1][PARKER ? T : 1];   // short-scan weights, one column per thread
+  unsigned pk_view = ~0u;                                 // the view they are of
   const int t = threadIdx.x, g = t / NP, j0 = t & (NP - 1);
-  const size_t ngroups = (nrows + 2 * G - 1) / (2 * G);
+  const size_t per_plane = (plane + 2 * G - 1) / (2 * G);
+  const size_t ngroups = PARKER ? nrows / plane * per_plane : (nrows + 2 * G - 1) / (2 * G);
+  const size_t t0 = PARKER ? ngroups * blockIdx.x / gridDim.x : blockIdx.x;
+  const size_t t1 = PARKER ? ngroups * (blockIdx.x + 1) / gridDim.x : ngroups;
+  const size_t step = PARKER ? 1 : gridDim.x;
 
   cf w[NT];
   fft_tw_load<N, 1, P, 0, NT>(w, j0, tw);
@@ -816,18 +830,23 @@ __global__ void __launch_bounds__(FftShape<LOG2N>::T) k_ramp_fft(
   auto rsrc = [](const float *p, size_t bytes) {
     return __builtin_amdgcn_make_buffer_rsrc((void *)p, (short)0, (int)bytes, 0x00020000);
   };
-  auto group_rows = [&](size_t gi) -> size_t {
-    const size_t r0 = gi * 2 * G;
-    return r0 >= nrows ? 0 : (nrows - r0 < 2 * (size_t)G ? nrows - r0 : 2 * (size_t)G);
-  };
   constexpr unsigned OOB = 0x80000000u;   // beyond any group's bytes
   const __amdgpu_buffer_rsrc_t rcos = rsrc(cosw, cosw ? (size_t)nv * nu * sizeof(float) : 0);
-  // raw rows and cosine weights of group gi
+  // first row and number of rows, raw rows and cosine weights of group gi (the
+  // PARKER groups are taken in order)
+  size_t row0 = 0, rows = 0;
+  size_t pk0 = PARKER ? t0 / per_plane * plane : 0, pv0 = PARKER ? t0 % per_plane * (2 * G) : 0;
   float x[2][H], cwv[2][H];
   auto fetch = [&](size_t gi) {
-    const __amdgpu_buffer_rsrc_t rin =
-        rsrc(in + gi * 2 * G * (size_t)nu, group_rows(gi) * nu * sizeof(float));
-    const unsigned v0 = (unsigned)((gi * 2 * G) % (size_t)nv);   // uniform
+    const size_t end = PARKER ? plane : nrows, first = PARKER ? pv0 : gi * 2 * G;
+    row0 = PARKER ? pk0 + pv0 : first;
+    rows = gi >= t1 ? 0 : (end - first < 2 * (size_t)G ? end - first : 2 * (size_t)G);
+    if constexpr (PARKER) {
+      pv0 += 2 * G;
+      if (pv0 >= plane) pv0 = 0, pk0 += plane;
+    }
+    const __amdgpu_buffer_rsrc_t rin = rsrc(in + row0 * (size_t)nu, rows * nu * sizeof(float));
+    const unsigned v0 = (unsigned)(row0 % (size_t)nv);   // uniform
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
       const int rl = 2 * g + h;   // row within the group
@@ -855,25 +874,33 @@ __global__ void __launch_bounds__(FftShape<LOG2N>::T) k_ramp_fft(
   // rows never waits for the previous group's stores (loads and stores
   // share one in-order counter).
   auto process = [&](size_t gi) __attribute__((always_inline)) {
-    const size_t ra = (gi * G + g) * 2;
-    const __amdgpu_buffer_rsrc_t rout =
-        rsrc(out + gi * 2 * G * (size_t)nu, group_rows(gi) * nu * sizeof(float));
+    const __amdgpu_buffer_rsrc_t rout = rsrc(out + row0 * (size_t)nu, rows * nu * sizeof(float));
     // the pair's weighted rows
     float xv[2][H];
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
-      const size_t r = ra + h;
-      float beta = 0.0f;
-      if (PARKER && r < nrows) beta = angles[r / (size_t)nv] * (3.14159265358979f / 180.0f);
+      bool have = true;
+      if constexpr (PARKER) {
+        const unsigned k0 = (unsigned)(row0 / (size_t)nv), v0 = (unsigned)(row0 - (size_t)k0 * nv);
+        const unsigned k = k0 + (v0 + (unsigned)(2 * g + h)) / (unsigned)nv;
+        have = (size_t)(2 * g + h) < rows;
+        if (have && k != pk_view) {
+          pk_view = k;
+          const float beta = angles[k] * (3.14159265358979f / 180.0f);
+#pragma unroll 1
+          for (int m = 0; m < H; ++m)
+            pkw[m][t] = parker_weight(j0 + m * NP, nu, beta, delta, tan_delta);
+        }
+      }
 #pragma unroll
       for (int m = 0; m < H; ++m) {
         float v = x[h][m];
         if (cosw) v *= cwv[h][m];
-        if (PARKER) v *= parker_weight(j0 + m * NP, nu, beta, delta, tan_delta);
+        if constexpr (PARKER) v *= have ? pkw[m][t] : 0.0f;
         xv[h][m] = v;
       }
     }
-    fetch(gi + gridDim.x);
+    fetch(gi + step);
     // their sums of squares over the pair's N/P threads (within one wave up
     // to 64): in FP32, and again in FP64 for a pair whose FP32 sums leave
     // [2^-100, 2^120] (tiny, huge, zero or not finite rows).  Only a power of
@@ -994,10 +1021,10 @@ __global__ void __launch_bounds__(FftShape<LOG2N>::T) k_ramp_fft(
         __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, -v.y * sc[1]), rout, ob, 0, 0);
       }
   };
-  fetch(blockIdx.x);
-  if ((size_t)blockIdx.x < ngroups) {
-    process(blockIdx.x);
-    for (size_t gi = (size_t)blockIdx.x + gridDim.x; gi < ngroups; gi += gridDim.x) process(gi);
+  fetch(t0);
+  if (t0 < t1) {
+    process(t0);
+    for (size_t gi = t0 + step; gi < t1; gi += step) process(gi);
   }
 }
 
@@ -1086,10 +1113,15 @@ int ensure_fft_tables(cbct_ctx ctx, int log2n) {
 std::atomic<int> g_fft_resident[2][FFT_MAX_LOG2N + 1];   // [parker][log2 N]
 
 template <int L>
-int launch_ramp_fft(cbct_ctx ctx, size_t ngroups, hipStream_t s, const float *in, float *out,
-                    size_t nrows, int nu, const float *tab, const float *cosw, int nv,
+int launch_ramp_fft(cbct_ctx ctx, hipStream_t s, const float *in, float *out, size_t nrows, int nu, const float *tab, const float *cosw, int nv,
                     const float *angles, int parker, float delta, float tan_delta) {
   const size_t N = size_t(1) << L;
+  constexpr size_t G2 = 2 * FftShape<L>::G;   // rows per group
+  // short scans: groups of one view where that fills the last group of each
+  // view with no more than an eighth of all rows, else across the views
+  const size_t whole = ((size_t)nv + G2 - 1) / G2 * G2;
+  const size_t plane = parker && nrows % nv == 0 && whole - nv <= (size_t)nv / 8 ? nv : nrows;
+  const size_t ngroups = (plane + G2 - 1) / G2 * (nrows / plane);
   const int pk = parker ? 1 : 0;
   int resident = g_fft_resident[pk][L].load();
   if (resident == 0) {
@@ -1105,15 +1137,13 @@ int launch_ramp_fft(cbct_ctx ctx, size_t ngroups, hipStream_t s, const float *in
     g_fft_resident[pk][L].store(resident);
   }
   const unsigned nb = (unsigned)(ngroups < (size_t)resident ? ngroups : (size_t)resident);
-  // the short-scan weights (Parker) only in their own instantiation: their
-  // range reductions would otherwise set the common kernel's register count
   if (parker)
     hipLaunchKernelGGL((k_ramp_fft<L, true>), dim3(nb), dim3(FftShape<L>::T), 0, s, in, out, nrows,
-                       nu, reinterpret_cast<const cf *>(tab), tab + 2 * N, cosw, nv, angles, delta,
+                       plane, nu, reinterpret_cast<const cf *>(tab), tab + 2 * N, cosw, nv, angles, delta,
                        tan_delta);
   else
     hipLaunchKernelGGL((k_ramp_fft<L, false>), dim3(nb), dim3(FftShape<L>::T), 0, s, in, out, nrows,
-                       nu, reinterpret_cast<const cf *>(tab), tab + 2 * N, cosw, nv, angles, delta,
+                       plane, nu, reinterpret_cast<const cf *>(tab), tab + 2 * N, cosw, nv, angles, delta,
                        tan_delta);
   return CBCT_OK;
 }
@@ -1130,19 +1160,17 @@ int run_ramp_fft(cbct_ctx ctx, int nu, int nv, size_t nrows, const float *in, fl
     return run_toeplitz_mfma(ctx, nu, nv, nrows, in, out, cosw, angles, parker, delta, tan_delta, s);
   int rc = ensure_fft_tables(ctx, L);
   if (rc) return rc;
-  const size_t rows_per_group = 2 * (size_t)(L >= 11 ? 1 : 2048 >> L);
-  const size_t ng = (nrows + rows_per_group - 1) / rows_per_group;
   const float *tab = ctx->d_fft;
   cbct_prof_mark(ctx, PROF_FILTER, 0, s);
   switch (L) {
-    case 6: rc = launch_ramp_fft<6>(ctx, ng, s, in, out, nrows, nu, tab, cosw, nv, angles, parker, delta, tan_delta); break;
-    case 7: rc = launch_ramp_fft<7>(ctx, ng, s, in, out, nrows, nu, tab, cosw, nv, angles, parker, delta, tan_delta); break;
-    case 8: rc = launch_ramp_fft<8>(ctx, ng, s, in, out, nrows, nu, tab, cosw, nv, angles, parker, delta, tan_delta); break;
-    case 9: rc = launch_ramp_fft<9>(ctx, ng, s, in, out, nrows, nu, tab, cosw, nv, angles, parker, delta, tan_delta); break;
-    case 10: rc = launch_ramp_fft<10>(ctx, ng, s, in, out, nrows, nu, tab, cosw, nv, angles, parker, delta, tan_delta); break;
-    case 11: rc = launch_ramp_fft<11>(ctx, ng, s, in, out, nrows, nu, tab, cosw, nv, angles, parker, delta, tan_delta); break;
-    case 12: rc = launch_ramp_fft<12>(ctx, ng, s, in, out, nrows, nu, tab, cosw, nv, angles, parker, delta, tan_delta); break;
-    default: rc = launch_ramp_fft<13>(ctx, ng, s, in, out, nrows, nu, tab, cosw, nv, angles, parker, delta, tan_delta); break;
+    case 6: rc = launch_ramp_fft<6>(ctx, s, in, out, nrows, nu, tab, cosw, nv, angles, parker, delta, tan_delta); break;
+    case 7: rc = launch_ramp_fft<7>(ctx, s, in, out, nrows, nu, tab, cosw, nv, angles, parker, delta, tan_delta); break;
+    case 8: rc = launch_ramp_fft<8>(ctx, s, in, out, nrows, nu, tab, cosw, nv, angles, parker, delta, tan_delta); break;
+    case 9: rc = launch_ramp_fft<9>(ctx, s, in, out, nrows, nu, tab, cosw, nv, angles, parker, delta, tan_delta); break;
+    case 10: rc = launch_ramp_fft<10>(ctx, s, in, out, nrows, nu, tab, cosw, nv, angles, parker, delta, tan_delta); break;
+    case 11: rc = launch_ramp_fft<11>(ctx, s, in, out, nrows, nu, tab, cosw, nv, angles, parker, delta, tan_delta); break;
+    case 12: rc = launch_ramp_fft<12>(ctx, s, in, out, nrows, nu, tab, cosw, nv, angles, parker, delta, tan_delta); break;
+    default: rc = launch_ramp_fft<13>(ctx, s, in, out, nrows, nu, tab, cosw, nv, angles, parker, delta, tan_delta); break;
   }
   if (rc) return rc;
   cbct_prof_mark(ctx, PROF_FILTER, 1, s);
