@@ -1033,14 +1033,23 @@ std::vector<double> spatial_kernel(int nu, const float *F) {
   std::vector<double> h(nu);
   const double pi = 3.14159265358979323846;
   const double inv = 1.0 / (2.0 * nu);
-  for (int m = 0; m < nu; ++m) {
-    double acc = (double)F[0] + (double)F[nu] * ((m & 1) ? -1.0 : 1.0);
-    for (int k = 1; k < nu; ++k) {
-      // reduce k*m mod 2nu exactly before taking the cosine
-      const long long km = ((long long)k * m) % (2LL * nu);
-      acc += 2.0 * (double)F[k] * std::cos(pi * (double)km / nu);
-    }
-    h[m] = acc * inv;
+  // cos(pi k m / nu) by k m mod 2nu, exactly reduced: 2nu cosines instead of
+  // nu^2 (0.8 ms of a reconstruction at nu = 256).  Four m at a time, each with
+  // its own sum in the order of k: one sum is a chain of additions.
+  std::vector<double> cs(2 * (size_t)nu);
+  for (int q = 0; q < 2 * nu; ++q) cs[q] = std::cos(pi * (double)q / nu);
+  for (int m0 = 0; m0 < nu; m0 += 4) {
+    double acc[4];
+    int km[4] = {0, 0, 0, 0};
+    for (int i = 0; i < 4; ++i) acc[i] = (double)F[0] + (double)F[nu] * ((i & 1) ? -1.0 : 1.0);
+    for (int k = 1; k < nu; ++k)
+      for (int i = 0; i < 4; ++i) {
+        const int m = m0 + i < nu ? m0 + i : 0;
+        km[i] += m;
+        if (km[i] >= 2 * nu) km[i] -= 2 * nu;
+        acc[i] += 2.0 * (double)F[k] * cs[km[i]];
+      }
+    for (int i = 0; i < 4 && m0 + i < nu; ++i) h[m0 + i] = acc[i] * inv;
   }
   return h;
 }
@@ -1090,19 +1099,26 @@ int ensure_fft_tables(cbct_ctx ctx, int log2n) {
     tab[2 * m + 1] = (float)-std::sin(2.0 * pi * (double)m / (double)N);
   }
   const std::vector<double> &h = ctx->h64;
-  for (size_t k = 0; k <= N / 2; ++k) {
-    double acc = h[0];
-    for (int t = 1; t < nu; ++t) acc += 2.0 * h[t] * cs[(k * (size_t)t) & (N - 1)];
-    tab[2 * N + k] = (float)(acc / (double)N);
-    tab[2 * N + ((N - k) & (N - 1))] = tab[2 * N + k];
+  for (size_t k0 = 0; k0 <= N / 2; k0 += 4) {   // four sums at a time, each in the order of t
+    double acc[4] = {h[0], h[0], h[0], h[0]};
+    for (int t = 1; t < nu; ++t)
+      for (size_t i = 0; i < 4; ++i) acc[i] += 2.0 * h[t] * cs[((k0 + i) * (size_t)t) & (N - 1)];
+    for (size_t k = k0; k < k0 + 4 && k <= N / 2; ++k) {
+      tab[2 * N + k] = (float)(acc[k - k0] / (double)N);
+      tab[2 * N + ((N - k) & (N - 1))] = tab[2 * N + k];
+    }
   }
   if (ctx->d_fft) {
     int rc = cbct_wait_tables(ctx);
     if (rc) return rc;
-    (void)hipFree(ctx->d_fft);
-    ctx->d_fft = nullptr;
+    ctx->fft_log2n = 0;
+    if (ctx->fft_alloc_log2n != log2n) {
+      (void)hipFree(ctx->d_fft);
+      ctx->d_fft = nullptr;
+    }
   }
-  CBCT_HIP_CHECK(ctx, hipMalloc(&ctx->d_fft, sizeof(float) * tab.size()));
+  if (!ctx->d_fft) CBCT_HIP_CHECK(ctx, hipMalloc(&ctx->d_fft, sizeof(float) * tab.size()));
+  ctx->fft_alloc_log2n = log2n;
   int rc = cbct_upload(ctx, ctx->d_fft, tab.data(), sizeof(float) * tab.size());
   if (rc) return rc;
   ctx->fft_log2n = log2n;
@@ -1245,16 +1261,18 @@ int cbct_filter_set(cbct_ctx ctx, int nu, const float *F) {
   // calls still reading the old tables finish first
   rc = cbct_wait_tables(ctx);
   if (rc) return rc;
-  if (ctx->d_h) (void)hipFree(ctx->d_h);
+  // (their memory is kept where the new ones are of the same size)
+  if (ctx->d_h && ctx->h64.size() != (size_t)nu) {
+    (void)hipFree(ctx->d_h);
+    ctx->d_h = nullptr;
+  }
   if (ctx->d_thi) (void)hipFree(ctx->d_thi);
   if (ctx->d_tlo) (void)hipFree(ctx->d_tlo);
-  if (ctx->d_fft) (void)hipFree(ctx->d_fft);
-  ctx->d_h = nullptr;
   ctx->d_thi = ctx->d_tlo = nullptr;
-  ctx->d_fft = nullptr;
+  ctx->fft_log2n = 0;
   ctx->filter_nu = 0;
   ctx->h64 = h;
-  CBCT_HIP_CHECK(ctx, hipMalloc(&ctx->d_h, sizeof(float) * hm.size()));
+  if (!ctx->d_h) CBCT_HIP_CHECK(ctx, hipMalloc(&ctx->d_h, sizeof(float) * hm.size()));
   rc = cbct_upload(ctx, ctx->d_h, hm.data(), sizeof(float) * hm.size());
   if (rc) return rc;
   ctx->filter_nu = nu;

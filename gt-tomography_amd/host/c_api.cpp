@@ -129,8 +129,7 @@ int gtt_fdk_reconstruct_3d(const cbct_geom *g, const float *angles, const float 
     Scan s = make_scan(g, angles, offsets, nviews, bin_index, bin_sizes, nbins, projections, true);
     std::shared_ptr<std::vector<float>> F;
     if (filter) F = std::make_shared<std::vector<float>>(filter, filter + g->nu + 1);
-    FDKResult r = FDK_reconstruct_3d(s.acq, s.binning, s.vol_dims, s.dims_mm, F, spp);
-    std::memcpy(volume_out, r.image->get_data_ptr(), r.image->get_number_of_bytes());
+    FDKResult r = fdk_reconstruct_3d_into(s.acq, s.binning, s.vol_dims, s.dims_mm, F, spp, volume_out);
     if (scale_out) *scale_out = r.scale;
   });
 }

@@ -4,10 +4,16 @@
 
 #include <hip/hip_runtime_api.h>
 
+#include <algorithm>
+#include <atomic>
+#include <cstring>
 #include <map>
+#include <mutex>
 #include <set>
-#include <vector>
 #include <string>
+#include <system_error>
+#include <thread>
+#include <vector>
 
 namespace gtt {
 
@@ -87,8 +93,13 @@ void release_context(cbct_ctx c) {
   t_pool[it->second].push_back(c);
 }
 
+namespace {
+void free_idle_slots();
+}
+
 void release_thread_resources() {
   trim_device_cache();
+  free_idle_slots();
   for (auto &kv : t_pool)
     for (cbct_ctx c : kv.second) cbct_ctx_destroy(c);
   t_pool.clear();
@@ -136,6 +147,7 @@ size_t retained_device_bytes() {
 
 void trim_thread_memory() {
   trim_device_cache();
+  free_idle_slots();
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess) return;
   auto it = t_ctx.find(dev);
@@ -266,13 +278,165 @@ PrivateStream::~PrivateStream() {
 void copy_d2d(void *dst, const void *src, size_t bytes) {
   hip_check(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToDevice, t_stream), "hipMemcpyAsync");
 }
+
+// Copies between the device and pageable host memory go through pinned slots:
+// COPY_THREADS threads, each with two slots, take chunks in turn and copy one
+// slot on the host while the other is on the bus.  The runtime's own path
+// copies on one thread.  To the device: 35 MB 1.39 -> 1.03 ms (0.65 on the bus
+// alone), 16 MB 0.68 -> 0.57, 8 MB 0.34 -> 0.37.  Back, into fresh memory: 35 MB
+// 3.66 -> 1.45 ms, 8 MB 0.48 -> 0.36, 4 MB 0.24 -> 0.22.  So from 16 MB on and from
+// 4 MB on; smaller copies, and those whose host side is pinned already, keep
+// the runtime's path, and so does everything if no pinned memory can be had.
+namespace {
+constexpr size_t COPY_SLOT = size_t(4) << 20, COPY_MIN_H2D = size_t(16) << 20,
+                 COPY_MIN_D2H = size_t(4) << 20;
+constexpr int COPY_THREADS = 4;
+
+// Slots and events of one copy in flight, all of one device.
+struct CopySlots {
+  int device = 0;
+  char *mem = nullptr;   // 2 COPY_THREADS slots
+  hipEvent_t done[2 * COPY_THREADS] = {};
+  ~CopySlots() {
+    for (hipEvent_t e : done)
+      if (e) (void)hipEventDestroy(e);
+    if (mem) (void)hipHostFree(mem);
+  }
+};
+// Idle slots, at most COPY_IDLE sets (32 MB each), for any thread's next copy;
+// trim_thread_memory and release_thread_resources free them.
+constexpr size_t COPY_IDLE = 2;
+std::mutex g_copy_mu;
+std::vector<CopySlots *> &copy_idle() {   // never destroyed: the runtime may be gone by then
+  static auto *v = [] {
+    auto *n = new std::vector<CopySlots *>;
+    n->reserve(COPY_IDLE);
+    return n;
+  }();
+  return *v;
+}
+
+CopySlots *take_slots(int dev) {
+  {
+    std::lock_guard<std::mutex> lk(g_copy_mu);
+    auto &v = copy_idle();
+    for (size_t i = 0; i < v.size(); ++i)
+      if (v[i]->device == dev) {
+        CopySlots *c = v[i];
+        v.erase(v.begin() + i);
+        return c;
+      }
+  }
+  auto *c = new CopySlots;
+  c->device = dev;
+  bool ok = hipHostMalloc(reinterpret_cast<void **>(&c->mem), 2 * COPY_THREADS * COPY_SLOT, 0) == hipSuccess;
+  for (hipEvent_t &e : c->done) ok = ok && hipEventCreateWithFlags(&e, hipEventDisableTiming) == hipSuccess;
+  if (ok) return c;
+  (void)hipGetLastError();
+  delete c;
+  return nullptr;
+}
+
+void give_slots(CopySlots *c) {
+  {
+    std::lock_guard<std::mutex> lk(g_copy_mu);
+    if (copy_idle().size() < COPY_IDLE) {
+      copy_idle().push_back(c);
+      return;
+    }
+  }
+  delete c;
+}
+
+void free_idle_slots() {
+  std::vector<CopySlots *> v;
+  {
+    std::lock_guard<std::mutex> lk(g_copy_mu);
+    v.swap(copy_idle());
+  }
+  for (CopySlots *c : v) delete c;
+}
+
+bool pageable(const void *host) {
+  hipPointerAttribute_t a{};
+  if (hipPointerGetAttributes(&a, host) != hipSuccess) {
+    (void)hipGetLastError();
+    return true;
+  }
+  return a.type == hipMemoryTypeUnregistered;
+}
+
+// The copy through slots; false if it has to take the runtime's path.  Waits
+// for the stream, also after an error, before the slots are given back.
+bool copy_through_slots(char *dev, char *host, size_t bytes, bool to_device) {
+  int d = 0;
+  if (bytes < (to_device ? COPY_MIN_H2D : COPY_MIN_D2H) || hipGetDevice(&d) != hipSuccess || !pageable(host)) return false;
+  CopySlots *c = take_slots(d);
+  if (!c) return false;
+  const hipStream_t s = t_stream;
+  // an eighth of the copy, but 1 MB to a slot: each chunk costs about 14 us more
+  // than its time on the bus, and a last copy on the host is not hidden
+  const size_t eighth = (bytes / (2 * COPY_THREADS) + 4095) / 4096 * 4096;
+  const size_t chunk = std::min(COPY_SLOT, std::max(size_t(1) << 20, eighth));
+  const size_t chunks = (bytes + chunk - 1) / chunk;
+  std::atomic<size_t> next{0};
+  std::atomic<int> error{(int)hipSuccess};
+  auto work = [&](int t) {
+    size_t at[2] = {chunks, chunks};   // the chunk in each slot (chunks: none)
+    auto len = [&](size_t k) { return std::min(chunk, bytes - k * chunk); };
+    auto run = [&]() -> hipError_t {
+      hipError_t e = hipSetDevice(d);
+      for (int i = 0; e == hipSuccess; i ^= 1) {
+        char *slot = c->mem + (2 * t + i) * COPY_SLOT;
+        if (at[i] < chunks) {   // the slot's last chunk has left it or come in
+          if ((e = hipEventSynchronize(c->done[2 * t + i])) != hipSuccess) break;
+          if (!to_device) std::memcpy(host + at[i] * chunk, slot, len(at[i]));
+          at[i] = chunks;
+        }
+        const size_t k = error.load() == (int)hipSuccess ? next.fetch_add(1) : chunks;
+        if (k >= chunks) {
+          if (at[i ^ 1] >= chunks) break;   // both slots idle
+          continue;
+        }
+        if (to_device) std::memcpy(slot, host + k * chunk, len(k));
+        e = to_device ? hipMemcpyAsync(dev + k * chunk, slot, len(k), hipMemcpyHostToDevice, s)
+                      : hipMemcpyAsync(slot, dev + k * chunk, len(k), hipMemcpyDeviceToHost, s);
+        if (e == hipSuccess) e = hipEventRecord(c->done[2 * t + i], s);
+        at[i] = k;
+      }
+      return e;
+    };
+    const hipError_t e = run();
+    int none = (int)hipSuccess;
+    if (e != hipSuccess) error.compare_exchange_strong(none, (int)e);
+  };
+  std::thread helpers[COPY_THREADS];
+  try {
+    for (int t = 1; t < COPY_THREADS; ++t) helpers[t] = std::thread(work, t);
+  } catch (const std::system_error &) {   // no more threads: those there are share the chunks
+  }
+  work(0);
+  for (auto &h : helpers)
+    if (h.joinable()) h.join();
+  const hipError_t e = hipStreamSynchronize(s);
+  give_slots(c);
+  hip_check((hipError_t)error.load(), to_device ? "hipMemcpyAsync H2D" : "hipMemcpyAsync D2H");
+  hip_check(e, "hipStreamSynchronize");
+  return true;
+}
+}  // namespace
+
 // Host copies are ordered after the thread's queued work and complete before
 // returning (the host buffer may be reused or read right away).
 void copy_h2d(void *dst, const void *src, size_t bytes) {
+  if (copy_through_slots(static_cast<char *>(dst), static_cast<char *>(const_cast<void *>(src)), bytes, true))
+    return;
   hip_check(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, t_stream), "hipMemcpyAsync H2D");
   hip_check(hipStreamSynchronize(t_stream), "hipStreamSynchronize");
 }
 void copy_d2h(void *dst, const void *src, size_t bytes) {
+  if (copy_through_slots(static_cast<char *>(const_cast<void *>(src)), static_cast<char *>(dst), bytes, false))
+    return;
   hip_check(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, t_stream), "hipMemcpyAsync D2H");
   hip_check(hipStreamSynchronize(t_stream), "hipStreamSynchronize");
 }

@@ -8,6 +8,7 @@
 
 #include "cbct.h"
 #include "gtt/CBCT_acquisition.h"
+#include "gtt/fdk.h"
 
 namespace gtt {
 
@@ -64,5 +65,13 @@ inline Scan make_scan(const cbct_geom *g, const float *angles, const float *offs
   if (nbins > 1) s.vol_dims.push_back((size_t)nbins);
   return s;
 }
+
+// FDK_reconstruct_3d with the result straight into `volume` (the result's image
+// wraps it) unless that is null.
+FDKResult fdk_reconstruct_3d_into(std::shared_ptr<CBCT_acquisition> acquisition,
+                                  std::shared_ptr<CBCT_binning> binning,
+                                  const std::vector<size_t> &is_dims, floatd3 is_dims_in_mm,
+                                  std::shared_ptr<std::vector<float>> frequency_filter,
+                                  float samples_per_pixel, float *volume);
 
 }  // namespace gtt

@@ -116,8 +116,7 @@ void run_request(Job &j) {
     std::shared_ptr<std::vector<float>> F;
     if (r.filter) F = std::make_shared<std::vector<float>>(r.filter, r.filter + r.geom.nu + 1);
     const float spp = r.samples_per_pixel > 0 ? r.samples_per_pixel : 1.5f;
-    FDKResult out = FDK_reconstruct_3d(s.acq, s.binning, s.vol_dims, s.dims_mm, F, spp);
-    std::memcpy(r.volume_out, out.image->get_data_ptr(), out.image->get_number_of_bytes());
+    FDKResult out = fdk_reconstruct_3d_into(s.acq, s.binning, s.vol_dims, s.dims_mm, F, spp, r.volume_out);
     j.scale = out.scale;
   } else {
     if (r.subsets <= 0) throw std::runtime_error("number of subsets must be positive");
