@@ -172,12 +172,12 @@ __global__ void __launch_bounds__(BP_TX *BP_TY) k_bp(BPParams P, const ViewF *__
 }
 
 // LDS-staged backprojector.  Per view, each block's detector rectangle
-// (k_bpp_rects) is copied into LDS by 16-byte direct global-to-LDS loads, one
+// (bpp_rect) is copied into LDS by 16-byte direct global-to-LDS loads, one
 // view ahead, and every voxel takes its taps from there.  Two layouts, both
 // 4-byte elements in rows of pnu2 (16-byte aligned): PAIRS (BF16 working
-// copies, k_pad_staged): element (a, b) holds the taps (a, b) and (a+1, b), so
+// copies, pad_staged): element (a, b) holds the taps (a, b) and (a+1, b), so
 // the four taps of a voxel-view are two elements one LDS row apart, one
-// ds_read2_b32; plain FP32 (k_pad_staged): the four taps are two adjacent
+// ds_read2_b32; plain FP32 (pad_staged): the four taps are two adjacent
 // pairs of elements one row apart, two ds_read2_b32.  Views whose rectangle
 // does not fit read the copy directly.  Same arithmetic, same bits as k_bp.
 //
@@ -209,11 +209,10 @@ constexpr int bpp_waves(bool pairs, bool fbp, int rw) {
 // right tap's); u0 is rounded down to 4 elements so the copies are 16-byte
 // aligned.
 template <int KZ>
-__global__ void __launch_bounds__(256) k_bpp_rects(BPParams P, const ViewF *__restrict__ views,
-                                                   uint2 *__restrict__ rects, unsigned gx, unsigned gy,
-                                                   unsigned nblocks) {
+__device__ __forceinline__ void bpp_rect(const BPParams &P, const ViewF *__restrict__ views,
+                                         uint2 *__restrict__ rects, unsigned gx, unsigned gy,
+                                         unsigned nblocks, size_t t) {
 #pragma clang fp contract(off)
-  const size_t t = (size_t)blockIdx.x * 256 + threadIdx.x;
   if (t >= (size_t)nblocks * P.nviews) return;
   const unsigned L = (unsigned)(t / P.nviews), k = (unsigned)(t % P.nviews);
   const int xb = (int)(L % gx) * BP_TX, yb = (int)((L / gx) % gy) * BP_TY;
@@ -503,16 +502,16 @@ inline dim3 pad_grid(unsigned pnu, int nviews) {
 // (one 16-byte store) from the projection values at u = a0-1 .. a0+3: one
 // 16-byte (FP32) or 8-byte (BF16) load plus the value before when the group
 // lies inside the row and vec (rows aligned for it) is set, else value by
-// value.  Grid as k_pad_quad over pnu2 / 4 columns.
+// value.  Block (bx, by, bz) of a grid as k_pad_quad's over pnu2 / 4 columns.
 template <typename TI, bool PAIRS>
-__global__ void __launch_bounds__(256) k_pad_staged(const TI *__restrict__ in, unsigned *__restrict__ out,
-                                                    int nu, int nv, unsigned pnu2, unsigned pnv,
-                                                    int nviews, int vec) {
-  const int a0 = 4 * (int)(blockIdx.x * 64 + (threadIdx.x & 63));
+__device__ __forceinline__ void pad_staged(const TI *__restrict__ in, unsigned *__restrict__ out, int nu,
+                                           int nv, unsigned pnu2, unsigned pnv, int nviews, int vec,
+                                           uint3 at, uint3 grid) {
+  const int a0 = 4 * (int)(at.x * 64 + (threadIdx.x & 63));
   if (a0 >= (int)pnu2) return;
-  const int b0 = (int)(blockIdx.y * 4 + (threadIdx.x >> 6)), bs = (int)(gridDim.y * 4);
+  const int b0 = (int)(at.y * 4 + (threadIdx.x >> 6)), bs = (int)(grid.y * 4);
   const bool inner = vec && a0 >= 4 && a0 + 3 < nu;
-  for (int k = (int)blockIdx.z; k < nviews; k += (int)gridDim.z) {
+  for (int k = (int)at.z; k < nviews; k += (int)grid.z) {
     const TI *pk = in + (size_t)nu * nv * k;
     unsigned *ok = out + (size_t)pnu2 * pnv * k;
     for (int b = b0; b < (int)pnv; b += bs) {
@@ -551,6 +550,26 @@ __global__ void __launch_bounds__(256) k_pad_staged(const TI *__restrict__ in, u
       *reinterpret_cast<uint4 *>(ok + (size_t)pnu2 * b + a0) = o;
     }
   }
+}
+
+// What the staged kernel needs, in one launch: the rectangles (the first
+// rect_blocks blocks) beside the copies, which are bound by memory (copies
+// 1.04 ms and rectangles 0.17 ms at 512^3, 720 views) or, in a subset of few
+// views, by the launches themselves: a call of 64^3, 9 views 22.6 -> 20.1 us,
+// 128^3, 20 views 37.3 -> 35.2, 256^3, 36 views 198 -> 196; large ones equal.
+template <typename TI, bool PAIRS, int Z>
+__global__ void __launch_bounds__(256) k_bpp_prep(BPParams P, const ViewF *__restrict__ views,
+                                                  uint2 *__restrict__ rects, unsigned gx, unsigned gy,
+                                                  unsigned nblocks, unsigned rect_blocks,
+                                                  const TI *__restrict__ in, unsigned *__restrict__ out,
+                                                  int nu, int nv, int vec, uint3 pad) {
+  if (blockIdx.x < rect_blocks) {
+    bpp_rect<Z>(P, views, rects, gx, gy, nblocks, (size_t)blockIdx.x * 256 + threadIdx.x);
+    return;
+  }
+  const unsigned b = blockIdx.x - rect_blocks, yz = b / pad.x;
+  pad_staged<TI, PAIRS>(in, out, nu, nv, P.pnu2, P.pnv, P.nviews, vec,
+                        make_uint3(b % pad.x, yz % pad.y, yz / pad.y), pad);
 }
 
 // Space carver (xray/conebeam_projection.cu:822-921): nearest-texel lookups,
@@ -762,22 +781,14 @@ int run_bp(cbct_ctx ctx, const cbct_geom *g, BPParams P, dim3 grid, int kz, int 
     unsigned *cp = static_cast<unsigned *>(ctx->ws->proj_pad.ptr);
     uint2 *rects = static_cast<uint2 *>(ctx->ws->bp_rects.ptr);
     const int vec = g->nu % 4 == 0 && reinterpret_cast<uintptr_t>(proj) % (4 * sizeof(TI)) == 0;
-    if (sizeof(T) == 2)
-      hipLaunchKernelGGL((k_pad_staged<TI, true>), pad_grid(P.pnu2 / 4, nviews), dim3(256), 0, s, proj, cp,
-                         g->nu, g->nv, P.pnu2, P.pnv, nviews, vec);
-    else
-      hipLaunchKernelGGL((k_pad_staged<TI, false>), pad_grid(P.pnu2 / 4, nviews), dim3(256), 0, s, proj,
-                         cp, g->nu, g->nv, P.pnu2, P.pnv, nviews, vec);
-    CBCT_LAUNCH_CHECK(ctx, "k_pad_staged");
     const ViewF *vf = ctx->d_views_f + view0;
-    const size_t nr = nblocks * nviews;
-    if (kz == 8)
-      hipLaunchKernelGGL((k_bpp_rects<8>), dim3((unsigned)((nr + 255) / 256)), dim3(256), 0, s, P, vf, rects,
-                         grid.x, grid.y, (unsigned)nblocks);
-    else
-      hipLaunchKernelGGL((k_bpp_rects<KZ>), dim3((unsigned)((nr + 255) / 256)), dim3(256), 0, s, P, vf, rects,
-                         grid.x, grid.y, (unsigned)nblocks);
-    CBCT_LAUNCH_CHECK(ctx, "k_bpp_rects");
+    const dim3 pad = pad_grid(P.pnu2 / 4, nviews);
+    const size_t rect_blocks = (nblocks * nviews + 255) / 256, prep = rect_blocks + (size_t)pad.x * pad.y * pad.z;
+    const auto k_prep = kz == 8 ? k_bpp_prep<TI, PAIRS, 8> : k_bpp_prep<TI, PAIRS, KZ>;
+    hipLaunchKernelGGL(k_prep, dim3((unsigned)prep), dim3(256), 0, s, P, vf, rects, grid.x, grid.y,
+                       (unsigned)nblocks, (unsigned)rect_blocks, proj, cp, g->nu, g->nv, vec,
+                       make_uint3(pad.x, pad.y, pad.z));
+    CBCT_LAUNCH_CHECK(ctx, "k_bpp_prep");
     cbct_prof_mark(ctx, PROF_BP, 0, s);
     if (kz == 8)
       launch_bpp_rows<PAIRS, 8>(P, rows, grid, s, vf, cp, rects, vol, fbp, accumulate);
