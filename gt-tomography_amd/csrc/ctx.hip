@@ -4,6 +4,7 @@
 #include <cstdarg>
 #include <cstring>
 #include <mutex>
+#include <new>
 
 #include "cbct_internal.h"
 
@@ -83,10 +84,7 @@ void Workspace::free_buffers() {
 
 Workspace::~Workspace() {
   (void)hipSetDevice(device);
-  if (done) {
-    if (recorded) (void)hipEventSynchronize(done);
-    (void)hipEventDestroy(done);
-  }
+  if (done) (void)hipEventSynchronize(done->e);
   free_buffers();
 }
 
@@ -98,20 +96,27 @@ CallScope::CallScope(cbct_ctx c, hipStream_t st) : ctx(c), s(st) {
   }
   capturing = cs != hipStreamCaptureStatusNone;
   Workspace &w = *ctx->ws;
-  if (!capturing && w.recorded && w.last != s) (void)hipStreamWaitEvent(s, w.done, 0);
+  if (!capturing && w.done && w.last != s) (void)hipStreamWaitEvent(s, w.done->e, 0);
 }
 
 CallScope::~CallScope() {
   if (capturing) return;
-  Workspace &w = *ctx->ws;
-  if (!w.done && hipEventCreateWithFlags(&w.done, hipEventDisableTiming) != hipSuccess) w.done = nullptr;
-  if (!ctx->done && hipEventCreateWithFlags(&ctx->done, hipEventDisableTiming) != hipSuccess)
-    ctx->done = nullptr;
-  if (w.done && hipEventRecord(w.done, s) == hipSuccess) {
-    w.recorded = true;
-    w.last = s;
+  if (cbct_done_event(ctx, false) != hipSuccess || hipEventRecord(ctx->done->e, s) != hipSuccess) return;
+  ctx->done_recorded = true;
+  ctx->ws->done = ctx->done;
+  ctx->ws->last = s;
+}
+
+hipError_t cbct_done_event(cbct_ctx ctx, bool own) {
+  if (ctx->done && !(own && ctx->ws->done == ctx->done)) return hipSuccess;
+  try {
+    auto d = std::make_shared<CallEvent>();
+    const hipError_t e = hipEventCreateWithFlags(&d->e, hipEventDisableTiming | hipEventDisableSystemFence);
+    if (e == hipSuccess) ctx->done = std::move(d);
+    return e;
+  } catch (const std::bad_alloc &) {
+    return hipErrorOutOfMemory;
   }
-  if (ctx->done && hipEventRecord(ctx->done, s) == hipSuccess) ctx->done_recorded = true;
 }
 
 namespace {
@@ -131,7 +136,7 @@ int cbct_upload(cbct_ctx ctx, void *dst, const void *src, size_t bytes) {
 }
 
 int cbct_wait_tables(cbct_ctx ctx) {
-  if (ctx->done_recorded) CBCT_HIP_CHECK(ctx, hipEventSynchronize(ctx->done));
+  if (ctx->done_recorded) CBCT_HIP_CHECK(ctx, hipEventSynchronize(ctx->done->e));
   return CBCT_OK;
 }
 
@@ -178,7 +183,7 @@ int cbct_ctx_trim(cbct_ctx ctx) {
   if (!ctx) return CBCT_ERR_ARG;
   (void)hipSetDevice(ctx->device);
   Workspace &w = *ctx->ws;
-  if (w.recorded) (void)hipEventSynchronize(w.done);
+  if (w.done) (void)hipEventSynchronize(w.done->e);
   w.free_buffers();
   return CBCT_OK;
 }
@@ -190,7 +195,13 @@ int cbct_ctx_share_workspace(cbct_ctx ctx, cbct_ctx owner) {
                      ctx->device, owner->device);
   if (ctx->ws == owner->ws) return CBCT_OK;
   (void)hipSetDevice(ctx->device);
-  ctx->ws = owner->ws;   // the previous workspace goes when its last holder does
+  // the previous workspace keeps the event of this context's last call, which is
+  // over, and goes when its last holder does
+  int rc = cbct_wait_tables(ctx);
+  if (rc) return rc;
+  ctx->done.reset();
+  ctx->done_recorded = false;
+  ctx->ws = owner->ws;
   return CBCT_OK;
 }
 
@@ -246,7 +257,6 @@ int cbct_ctx_destroy(cbct_ctx ctx) {
   if (!ctx) return CBCT_OK;
   (void)hipSetDevice(ctx->device);
   (void)cbct_wait_tables(ctx);
-  if (ctx->done) (void)hipEventDestroy(ctx->done);
   for (auto &pair : ctx->ev)
     for (auto &e : pair)
       if (e) (void)hipEventDestroy(e);
@@ -316,7 +326,7 @@ int cbct_views_set(cbct_ctx ctx, const float *angles_deg, const float *offsets, 
   ctx->views_h = std::move(vf);
   ctx->bpp_fit_cache.clear();
   // the event that marks the end of the calls reading this table
-  if (!ctx->done) CBCT_HIP_CHECK(ctx, hipEventCreateWithFlags(&ctx->done, hipEventDisableTiming));
+  CBCT_HIP_CHECK(ctx, cbct_done_event(ctx, false));
   return CBCT_OK;
 }
 
