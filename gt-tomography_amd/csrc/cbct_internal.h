@@ -69,9 +69,13 @@ struct cbct_ctx_s {
   ViewF *d_views_f = nullptr;
   float *d_angles = nullptr;  // degrees, for the Parker weights
   std::shared_ptr<Workspace> ws;
-  // end of the last call that read this context's tables (views, filter)
+  // end of the last call that used the workspace, and of the last cbct_fp_noalloc
+  // (made with the view table, recorded by no other call): the calls that read
+  // this context's tables (views, filter)
   std::shared_ptr<CallEvent> done;
   bool done_recorded = false;
+  CallEvent noalloc_done;
+  bool noalloc_recorded = false;
   // filter state
   int filter_nu = 0;
   int filter_engine = 2;
@@ -116,14 +120,15 @@ struct cbct_ctx_s {
 struct CallScope {
   cbct_ctx ctx;
   hipStream_t s;
-  bool capturing = false;
+  bool capturing;
   CallScope(cbct_ctx c, hipStream_t st);
   ~CallScope();
 };
-// Creates ctx->done if there is none; an event that the workspace refers to is
-// left to it when `own` is set.
-hipError_t cbct_done_event(cbct_ctx ctx, bool own);
-// Wait (host) for the end of the last call that read the context's tables.
+// Creates ctx->done if there is none.
+hipError_t cbct_done_event(cbct_ctx ctx);
+// Whether work on s is being captured into a graph.
+bool cbct_capturing(hipStream_t s);
+// Wait (host) for the end of the calls that read the context's tables.
 int cbct_wait_tables(cbct_ctx ctx);
 // Host-to-device copy of a context's table, complete on return.  It goes
 // through a non-blocking stream of the library's own (one per device), not

@@ -88,30 +88,37 @@ Workspace::~Workspace() {
   free_buffers();
 }
 
-CallScope::CallScope(cbct_ctx c, hipStream_t st) : ctx(c), s(st) {
+bool cbct_capturing(hipStream_t s) {
   hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(s, &cs) != hipSuccess) {
     (void)hipGetLastError();
-    cs = hipStreamCaptureStatusNone;
+    return false;
   }
-  capturing = cs != hipStreamCaptureStatusNone;
+  return cs != hipStreamCaptureStatusNone;
+}
+
+CallScope::CallScope(cbct_ctx c, hipStream_t st) : ctx(c), s(st), capturing(cbct_capturing(st)) {
   Workspace &w = *ctx->ws;
   if (!capturing && w.done && w.last != s) (void)hipStreamWaitEvent(s, w.done->e, 0);
 }
 
 CallScope::~CallScope() {
   if (capturing) return;
-  if (cbct_done_event(ctx, false) != hipSuccess || hipEventRecord(ctx->done->e, s) != hipSuccess) return;
+  if (cbct_done_event(ctx) != hipSuccess || hipEventRecord(ctx->done->e, s) != hipSuccess) return;
   ctx->done_recorded = true;
   ctx->ws->done = ctx->done;
   ctx->ws->last = s;
 }
 
-hipError_t cbct_done_event(cbct_ctx ctx, bool own) {
-  if (ctx->done && !(own && ctx->ws->done == ctx->done)) return hipSuccess;
+namespace {
+constexpr unsigned CALL_EVENT_FLAGS = hipEventDisableTiming | hipEventDisableSystemFence;
+}
+
+hipError_t cbct_done_event(cbct_ctx ctx) {
+  if (ctx->done) return hipSuccess;
   try {
     auto d = std::make_shared<CallEvent>();
-    const hipError_t e = hipEventCreateWithFlags(&d->e, hipEventDisableTiming | hipEventDisableSystemFence);
+    const hipError_t e = hipEventCreateWithFlags(&d->e, CALL_EVENT_FLAGS);
     if (e == hipSuccess) ctx->done = std::move(d);
     return e;
   } catch (const std::bad_alloc &) {
@@ -137,6 +144,7 @@ int cbct_upload(cbct_ctx ctx, void *dst, const void *src, size_t bytes) {
 
 int cbct_wait_tables(cbct_ctx ctx) {
   if (ctx->done_recorded) CBCT_HIP_CHECK(ctx, hipEventSynchronize(ctx->done->e));
+  if (ctx->noalloc_recorded) CBCT_HIP_CHECK(ctx, hipEventSynchronize(ctx->noalloc_done.e));
   return CBCT_OK;
 }
 
@@ -291,6 +299,9 @@ int cbct_views_set(cbct_ctx ctx, const float *angles_deg, const float *offsets, 
     return cbct_fail(ctx, CBCT_ERR_ARG, "Error: cbct_views_set: illegal angle array provided");
   int rc = cbct_set_device(ctx);
   if (rc) return rc;
+  // the events that mark the end of the calls reading this table
+  CBCT_HIP_CHECK(ctx, cbct_done_event(ctx));
+  if (!ctx->noalloc_done.e) CBCT_HIP_CHECK(ctx, hipEventCreateWithFlags(&ctx->noalloc_done.e, CALL_EVENT_FLAGS));
   std::vector<ViewD> vd(n);
   std::vector<ViewF> vf(n);
   ctx->angles_deg.assign(angles_deg, angles_deg + n);
@@ -326,8 +337,6 @@ int cbct_views_set(cbct_ctx ctx, const float *angles_deg, const float *offsets, 
   ctx->nviews = n;
   ctx->views_h = std::move(vf);
   ctx->bpp_fit_cache.clear();
-  // the event that marks the end of the calls reading this table
-  CBCT_HIP_CHECK(ctx, cbct_done_event(ctx, false));
   return CBCT_OK;
 }
 

@@ -1678,10 +1678,12 @@ int cbct_fp_noalloc(cbct_ctx ctx, const cbct_geom *g, int view0, int nviews, con
   if (rc) return rc;
   hipStream_t s = as_stream(stream);
   rc = run_fp_dtype(ctx, g, P, view0, nviews, vol, dtype, proj, accumulate, s, spp, ptr);
-  // this call read the view table: a later cbct_views_set waits for it (on an
-  // event of its own: the workspace's last call is another)
-  if (rc == CBCT_OK && cbct_done_event(ctx, true) == hipSuccess && hipEventRecord(ctx->done->e, s) == hipSuccess)
-    ctx->done_recorded = true;
+  // this call read the view table: a later cbct_views_set waits for it.  On an
+  // event of its own, so that the end of the last call in the workspace stays
+  // marked; calls that share the scratch are in order, so the last one's end is
+  // the end of all
+  if (rc == CBCT_OK && !cbct_capturing(s) && hipEventRecord(ctx->noalloc_done.e, s) == hipSuccess)
+    ctx->noalloc_recorded = true;
   return rc;
 }
 
