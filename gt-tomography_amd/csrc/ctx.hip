@@ -203,13 +203,13 @@ int cbct_ctx_share_workspace(cbct_ctx ctx, cbct_ctx owner) {
                      ctx->device, owner->device);
   if (ctx->ws == owner->ws) return CBCT_OK;
   (void)hipSetDevice(ctx->device);
-  // the previous workspace goes when its last holder does, and keeps the event of
-  // this context's last call (waited for here, since the context lets go of it)
-  if (ctx->done && ctx->ws->done == ctx->done) {
-    (void)cbct_wait_tables(ctx);
-    ctx->done.reset();
-    ctx->done_recorded = false;
-  }
+  // Calls in the previous workspace may still read this context's tables, and
+  // none of the next workspace's events comes after them: they end here.  The
+  // previous workspace goes when its last holder does, and may keep the event.
+  int rc = cbct_wait_tables(ctx);
+  if (rc) return rc;
+  ctx->done.reset();
+  ctx->done_recorded = false;
   ctx->ws = owner->ws;
   return CBCT_OK;
 }

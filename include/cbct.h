@@ -76,7 +76,8 @@ int cbct_profile_read(cbct_ctx ctx, double *fp_ms, double *bp_ms, double *filter
 /* Frees the context's scratch (it regrows on demand), after the last call
  * that used it has finished. */
 int cbct_ctx_trim(cbct_ctx ctx);
-/* ctx drops its own scratch and uses owner's from now on (same device).  The
+/* ctx drops its own scratch and uses owner's from now on (same device), after
+ * the calls made on ctx so far have finished (waits on the host).  The
  * scratch lives until the last context holding it is destroyed.  Contexts
  * that share scratch are used from one host thread at a time; their calls
  * are ordered as calls on one context are (above).  Lets the many per-subset

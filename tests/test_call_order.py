@@ -46,3 +46,29 @@ assert fp_noalloc(h, g, 6, S2) == 0
 sim.hip_capture(S2, 0)
 assert count("launch") and count("record") == 0
 """)
+
+
+@pytest.mark.parametrize("between", [False, True])
+@pytest.mark.parametrize("table", ["filter", "views"])
+def test_tables_wait_for_calls_in_the_workspace_before(run, table, between):
+    """A table is replaced after the context's calls in the workspace that it had before
+    the present one, whether or not another context has used that one since."""
+    run(f"""
+g = geom(16, 16, 16, 32, 24)
+a, b, other = context(angles_full(6), filt=32), context(angles_full(6)), context()
+assert L.cbct_ctx_share_workspace(b, a) == 0
+sim.hip_log_clear()
+assert prefilter(a, g, 6, S1) == 0
+read = len(log())
+if {between}:
+    assert bp(b, g, 6, S2) == 0
+assert L.cbct_ctx_share_workspace(a, other) == 0
+assert fp(a, g, 6, S3) == 0
+rc = set_filter(a, 32) if {table!r} == "filter" else views(a, angles_full(6, start=3.0))
+assert rc == 0
+o = Order(log())
+late = [x for u in o.unwaited for x in u if x in log()[:read]]
+assert o.unwaited and not late, late
+# and the workspace's own last call is still waited for by its next one
+assert fp(b, g, 6, S1) == 0
+""")
