@@ -46,6 +46,10 @@ struct Workspace {
   int device = 0;
   DeviceBuffer vol_pad;     // padded / repacked volume for the forward projector
   DeviceBuffer vol_cells;   // forward projector: packed (x, y) corners of the volume copy
+                            // (optional: cbct_reserve_cells)
+  size_t cells_refused = 0;      // bytes that could not be had for it, or were given back; 0: none
+  bool cells_captured = false;   // a captured call uses it
+  std::vector<DeviceBuffer> cells_kept;   // outgrown ones that captured calls use
   DeviceBuffer proj_pad;    // padded projections for the backprojector
   DeviceBuffer red;         // reduction partials
   DeviceBuffer filt_tmp;    // filter staging
@@ -157,8 +161,13 @@ int cbct_fail(cbct_ctx ctx, int code, const char *fmt, ...);
       return cbct_fail((ctx), CBCT_ERR_HIP, "%s launch: %s", (what), hipGetErrorString(_e)); \
   } while (0)
 
-// Workspace growth (device current must be ctx->device).
+// Workspace growth (device current must be ctx->device).  Where memory is
+// short, the packed volume copy is given back first.
 int cbct_reserve(cbct_ctx ctx, DeviceBuffer &b, size_t bytes);
+// Room for the packed volume copy, if it can be had: a faster call, not one that
+// fails.  What was refused or given back is not tried again until a trim; under
+// capture nothing is allocated, and what a captured call uses is kept until then.
+bool cbct_reserve_cells(cbct_ctx ctx, size_t bytes, bool capturing);
 int cbct_set_device(cbct_ctx ctx);
 int cbct_check_geom(cbct_ctx ctx, const cbct_geom *g, const char *who);
 int cbct_check_views(cbct_ctx ctx, int view0, int nviews, const char *who);

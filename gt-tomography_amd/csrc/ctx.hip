@@ -49,6 +49,16 @@ int cbct_reserve(cbct_ctx ctx, DeviceBuffer &b, size_t bytes) {
   }
   size_t want = bytes < 256 ? 256 : bytes;
   hipError_t e = hipMalloc(&b.ptr, want);
+  Workspace &w = *ctx->ws;
+  if (e == hipErrorOutOfMemory && w.vol_cells.ptr && !w.cells_captured) {
+    // (no call uses it after reserving anything else)
+    if (w.done) (void)hipEventSynchronize(w.done->e);
+    (void)hipFree(w.vol_cells.ptr);
+    w.cells_refused = w.vol_cells.bytes;
+    w.vol_cells = DeviceBuffer();
+    (void)hipGetLastError();
+    e = hipMalloc(&b.ptr, want);
+  }
   if (e != hipSuccess) {
     b.ptr = nullptr;
     (void)hipGetLastError();
@@ -57,6 +67,34 @@ int cbct_reserve(cbct_ctx ctx, DeviceBuffer &b, size_t bytes) {
   }
   b.bytes = want;
   return CBCT_OK;
+}
+
+bool cbct_reserve_cells(cbct_ctx ctx, size_t bytes, bool capturing) {
+  Workspace &w = *ctx->ws;
+  DeviceBuffer &b = w.vol_cells;
+  if (!b.ptr || b.bytes < bytes) {
+    if (capturing || (w.cells_refused && bytes >= w.cells_refused)) return false;
+    if (w.cells_captured) {
+      try {
+        w.cells_kept.push_back(b);
+      } catch (const std::bad_alloc &) {
+        return false;
+      }
+      w.cells_captured = false;
+    } else if (b.ptr) {
+      (void)hipFree(b.ptr);
+    }
+    b = DeviceBuffer();
+    if (hipMalloc(&b.ptr, bytes) != hipSuccess) {
+      b.ptr = nullptr;
+      (void)hipGetLastError();
+      w.cells_refused = bytes;
+      return false;
+    }
+    b.bytes = bytes;
+  }
+  if (capturing) w.cells_captured = true;
+  return true;
 }
 
 int cbct_check_geom(cbct_ctx ctx, const cbct_geom *g, const char *who) {
@@ -80,6 +118,10 @@ void Workspace::free_buffers() {
     b->ptr = nullptr;
     b->bytes = 0;
   }
+  for (auto &b : cells_kept) (void)hipFree(b.ptr);
+  cells_kept.clear();
+  cells_refused = 0;
+  cells_captured = false;
 }
 
 Workspace::~Workspace() {
@@ -289,7 +331,9 @@ const char *cbct_last_error(cbct_ctx ctx) {
 size_t cbct_workspace_bytes(cbct_ctx ctx) {
   if (!ctx) return 0;
   const Workspace &w = *ctx->ws;
-  return w.vol_pad.bytes + w.vol_cells.bytes + w.proj_pad.bytes + w.red.bytes + w.filt_tmp.bytes + w.ssim_ws.bytes +
+  size_t kept = 0;
+  for (const auto &b : w.cells_kept) kept += b.bytes;
+  return kept + w.vol_pad.bytes + w.vol_cells.bytes + w.proj_pad.bytes + w.red.bytes + w.filt_tmp.bytes + w.ssim_ws.bytes +
          w.bp_rects.bytes;
 }
 

@@ -1400,7 +1400,7 @@ int run_fp(cbct_ctx ctx, const cbct_geom *g, const FPParams &P, int view0, int n
   if (choice.vg > 0) Q.vg = (unsigned)choice.vg;
   // without memory for the packed copy the column kernels take every ray
   Q.split = !ext && clip_split(ctx, g, P, view0, nviews, esz) &&
-            cbct_reserve(ctx, ctx->ws->vol_cells, 4 * npad * esz) == CBCT_OK;
+            cbct_reserve_cells(ctx, 4 * npad * esz, cbct_capturing(s));
   const unsigned nslots = ceil_div(P.nv, 64);
   const unsigned cell_bytes = (unsigned)(4 * npad * esz);
   T *cells = static_cast<T *>(ctx->ws->vol_cells.ptr);

@@ -72,3 +72,71 @@ assert o.unwaited and not late, late
 # and the workspace's own last call is still waited for by its next one
 assert fp(b, g, 6, S1) == 0
 """)
+
+
+SLAB = """
+# most rays of the slab leave through its top or bottom: 30 views take them from the
+# packed copy (four padded volumes), one view does not
+g = geom(64, 64, 16, 48, 48)
+CELLS = 4 * 67 * 67 * 32 * 4
+def clip():
+    n = sum("k_fp_clip" in l for l in log())
+    sim.hip_log_clear()
+    return n
+h = context(angles_full(30))
+live = lambda: ctypes.c_size_t.in_dll(sim, "hip_live").value
+"""
+
+
+def test_packed_copy_without_memory(run):
+    """A packed copy that cannot be had is done without: no error, no further try until a
+    trim."""
+    run(SLAB + """
+assert fp(h, g, 1, S1) == 0 and clip() == 0
+limit(live() + CELLS - 1)
+assert fp(h, g, 30, S1) == 0 and count("launch") and clip() == 0
+assert L.cbct_last_error(h) == b""
+assert fp(h, g, 30, S1) == 0 and count("malloc") == 0 and clip() == 0
+limit(1 << 40)
+assert fp(h, g, 30, S1) == 0 and count("malloc") == 0 and clip() == 0
+assert L.cbct_ctx_trim(h) == 0 and fp(h, g, 30, S1) == 0 and clip() > 0
+""")
+
+
+def test_packed_copy_is_given_back(run):
+    """Memory that a call needs takes the packed copy's place, once, after the call that
+    used it."""
+    run(SLAB + """
+assert fp(h, g, 30, S1) == 0 and clip() > 0
+limit(live() + 4096)
+assert bp(h, g, 30, S2) == 0, L.cbct_last_error(h)
+assert fp(h, g, 30, S1) == 0 and bp(h, g, 30, S1) == 0 and count("launch")
+assert sum(l.startswith("malloc %d" % CELLS) for l in log()) == 0
+sim.hip_log_clear()
+assert fp(h, g, 30, S1) == 0 and bp(h, g, 30, S1) == 0 and count("malloc") == count("free") == 0
+assert L.cbct_last_error(h) == b""
+""")
+
+
+def test_packed_copy_under_capture(run):
+    """No memory is taken under capture, and what a captured call uses is not given back."""
+    run(SLAB + """
+assert fp(h, g, 1, S1) == 0
+sim.hip_log_clear()
+sim.hip_capture(S1, 1)
+assert fp(h, g, 30, S1) == 0 and count("malloc") == 0 and count("launch") and clip() == 0
+sim.hip_capture(S1, 0)
+assert fp(h, g, 30, S1) == 0 and clip() > 0
+sim.hip_capture(S1, 1)
+assert fp(h, g, 30, S1) == 0 and count("malloc") == 0 and clip() > 0
+sim.hip_capture(S1, 0)
+limit(live() + 4096)
+assert bp(h, g, 30, S1) == -4 and count("free") == 0
+limit(1 << 40)
+wide = geom(200, 200, 20, 16, 16)                    # sizes the padded copy alone
+assert fp(h, wide, 1, S1) == 0 and clip() == 0
+held = L.cbct_workspace_bytes(h)
+assert fp(h, geom(80, 80, 20, 48, 48), 30, S1) == 0 and count("free") == 0 and clip() > 0
+assert L.cbct_workspace_bytes(h) == held + 4 * 83 * 83 * 32 * 4
+assert L.cbct_ctx_trim(h) == 0 and L.cbct_workspace_bytes(h) == 0
+""")
