@@ -92,6 +92,7 @@ struct cbct_ctx_s {
   int bp_kz = 0;                 // z-voxels per BP thread: 0 = chosen by size, else 8 or 16
   int fp_max_rpl = 0;            // column engine: most detector rows per lane; 0 = unset (8; engine 1: 12)
   int fp_view_group = 6;         // column engine: adjacent views launched together per column
+  bool fp_packed = true;         // cbct_fp may build the packed volume copy (clip_cells)
   int fp_force_variant = 0;      // autotuner trials: variant and tile forced when > 0
   int fp_force_rpl = 0;
   int fp_force_zc = 0;

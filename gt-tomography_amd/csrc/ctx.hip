@@ -265,6 +265,7 @@ int cbct_ctx_reset(cbct_ctx ctx) {
   ctx->bp_kz = d.bp_kz;
   ctx->fp_max_rpl = d.fp_max_rpl;
   ctx->fp_view_group = d.fp_view_group;
+  ctx->fp_packed = d.fp_packed;
   ctx->fp_force_variant = d.fp_force_variant;
   ctx->fp_force_rpl = d.fp_force_rpl;
   ctx->fp_force_zc = d.fp_force_zc;

@@ -42,6 +42,7 @@
 #include <vector>
 
 #include "cbct_internal.h"
+#include "fp_cells.h"
 
 // Working copy of cbct_fp_noalloc: device memory the library owns for the
 // life of the process (one copy per GPU, each at its own address), so that
@@ -939,7 +940,7 @@ k_fp_colc(FPParams P, const ViewD *__restrict__ views, const T *__restrict__ vt,
 
 // The rays that the column kernels with P.split leave out (those not shared),
 // from the packed copy: one wave per 64 rows of a detector column.  Used where
-// many rays are clipped (clip_split).
+// many rays are clipped (clip_cells).
 template <typename T>
 __global__ void __launch_bounds__(64) k_fp_clip(FPParams P, const ViewD *__restrict__ views,
                                                 const T *__restrict__ cells, float *__restrict__ proj,
@@ -1075,9 +1076,6 @@ inline dim3 stride_grid(size_t n) {
   return dim3((unsigned)b);
 }
 
-// z-fastest padded length: nz + 3 rounded up to 16 elements
-inline size_t zpadded(int nz) { return (padded_dim(nz) + 15) & ~size_t(15); }
-
 int make_params(cbct_ctx ctx, const cbct_geom *g, float spp, FPParams &P) {
   const float fn = spp * (float)g->nx;
   if (!(fn >= 1.0f) || fn > 1e6f)
@@ -1089,7 +1087,7 @@ int make_params(cbct_ctx ctx, const cbct_geom *g, float spp, FPParams &P) {
   P.ny = g->ny;
   P.nz = g->nz;
   const size_t px = padded_dim(g->nx), py = padded_dim(g->ny), pz = padded_dim(g->nz);
-  const size_t pzz = zpadded(g->nz);
+  const size_t pzz = fp_zpadded(g->nz);
   if (px * py * pzz >= (1ull << 32) - 1)
     return cbct_fail(ctx, CBCT_ERR_UNSUPPORTED, "Error: conebeam_forwards_projection: volume too large for 32-bit indexing");
   (void)pz;
@@ -1335,23 +1333,13 @@ size_t fp_working_bytes(cbct_ctx ctx, const cbct_geom *g, const FPParams &P, int
   return ((size_t)P.pzx * padded_dim(g->ny) + 1024) * esz;
 }
 
-// Whether the rays that leave through the top or bottom go to k_fp_clip: when
-// their samples (those of the rows that reach past the volume's height at its
-// far side, an upper bound) outweigh building the packed copy.  The copy costs
-// 20 bytes of traffic per voxel (4.4 ps), the packed loads save about 1.6 ps a
-// sample.  The copy must stay within a buffer's 4 GB.
-bool clip_split(cbct_ctx ctx, const cbct_geom *g, const FPParams &P, int view0, int nviews, size_t esz) {
-  if ((size_t)P.pzx * padded_dim(g->ny) * 4 * esz >= (1ull << 32) - 64) return false;
-  const double R = 0.5 * std::sqrt((double)g->lx * g->lx + (double)g->ly * g->ly);
-  const double vmax = 0.5 * g->lz * g->sdd / ((double)g->sad + R);   // heights up to here are never clipped
-  const double pitch = (double)g->fov_v / g->nv;
+// Bytes of the packed copy from which k_fp_clip takes the rays that leave through
+// the top or bottom; 0: they stay with the column kernels.
+size_t clip_cells(cbct_ctx ctx, const cbct_geom *g, const FPParams &P, int view0, int nviews, size_t esz) {
+  if (!ctx->fp_packed) return 0;
   double rows = 0.0;
-  for (int k = 0; k < nviews; ++k) {
-    const double off = ctx->offsets[2 * (size_t)(view0 + k) + 1];
-    rows += std::max(0.0, 0.5 * g->fov_v + off - vmax) / pitch + std::max(0.0, 0.5 * g->fov_v - off - vmax) / pitch;
-  }
-  const double samples = rows * g->nu * P.n, nvox = (double)g->nx * g->ny * g->nz;
-  return samples > 3.6 * nvox;
+  for (int k = 0; k < nviews; ++k) rows += fp_clipped_rows(g, ctx->offsets[2 * (size_t)(view0 + k) + 1]);
+  return fp_cells_bytes(g, rows, P.n, esz);
 }
 
 // TI: the caller's volume type; T: the padded working copy's type.  The
@@ -1399,10 +1387,9 @@ int run_fp(cbct_ctx ctx, const cbct_geom *g, const FPParams &P, int view0, int n
   FPParams Q = P;
   if (choice.vg > 0) Q.vg = (unsigned)choice.vg;
   // without memory for the packed copy the column kernels take every ray
-  Q.split = !ext && clip_split(ctx, g, P, view0, nviews, esz) &&
-            cbct_reserve_cells(ctx, 4 * npad * esz, cbct_capturing(s));
+  const size_t cell_bytes = ext ? 0 : clip_cells(ctx, g, P, view0, nviews, esz);
+  Q.split = cell_bytes && cbct_reserve_cells(ctx, cell_bytes, cbct_capturing(s));
   const unsigned nslots = ceil_div(P.nv, 64);
-  const unsigned cell_bytes = (unsigned)(4 * npad * esz);
   T *cells = static_cast<T *>(ctx->ws->vol_cells.ptr);
   if (Q.split) {
     hipLaunchKernelGGL(k_pack_cells<T>, dim3(std::min(ceil_div(npad / 4, 256), 65536u)), dim3(256), 0, s, vt, cells,
@@ -1418,7 +1405,7 @@ int run_fp(cbct_ctx ctx, const cbct_geom *g, const FPParams &P, int view0, int n
     for (int v0 = 0; v0 < nviews; v0 += max_views) {
       const unsigned nblocks = (unsigned)(per_view * (size_t)std::min(max_views, nviews - v0));
       hipLaunchKernelGGL(k_fp_clip<T>, dim3(nblocks), dim3(64), 0, s, Q, views + v0, cells,
-                         proj + (size_t)v0 * P.nu * P.nv, accumulate, nslots, nblocks, cell_bytes);
+                         proj + (size_t)v0 * P.nu * P.nv, accumulate, nslots, nblocks, (unsigned)cell_bytes);
     }
   }
   cbct_prof_mark(ctx, PROF_FP, 1, s);
@@ -1558,6 +1545,12 @@ int cbct_fp_tile(cbct_ctx ctx, int max_rows_per_lane) {
   if (max_rows_per_lane < 1 || max_rows_per_lane > 12)
     return cbct_fail(ctx, CBCT_ERR_ARG, "cbct_fp_tile: rows per lane %d outside 1..12", max_rows_per_lane);
   ctx->fp_max_rpl = max_rows_per_lane;
+  return CBCT_OK;
+}
+
+int cbct_fp_packed(cbct_ctx ctx, int on) {
+  if (!ctx) return CBCT_ERR_ARG;
+  ctx->fp_packed = on != 0;
   return CBCT_OK;
 }
 

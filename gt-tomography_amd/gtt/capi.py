@@ -110,6 +110,7 @@ def load():
         "cbct_fp_autotune_clear": (I, []),
         "cbct_fp_tile": (I, [P, I]),
         "cbct_fp_view_group": (I, [P, I]),
+        "cbct_fp_packed": (I, [P, I]),
         "cbct_bp_engine": (I, [P, I]),
         "cbct_bp_kernel": (ctypes.c_char_p, [P, G, I, I]),
         "cbct_bp_kz": (I, [P, I]),
@@ -308,6 +309,10 @@ class Context:
     def fp_view_group(self, views):
         """Column engine: adjacent views launched together per detector column (1..64)."""
         self._check(self.lib.cbct_fp_view_group(self.h, int(views)))
+
+    def fp_packed(self, on):
+        """Whether fp may hold a packed copy of the volume for clipped rays (default on)."""
+        self._check(self.lib.cbct_fp_packed(self.h, int(on)))
 
     def bp_engine(self, engine):
         """2 = default (LDS-staged kernel where its tile holds the blocks'

@@ -24,6 +24,7 @@ namespace {
 thread_local std::map<int, cbct_ctx> t_ctx;
 thread_local hipStream_t t_stream = nullptr;
 thread_local int t_storage = CBCT_F32;
+thread_local bool t_packed = true;
 thread_local bool t_autotune = false;
 thread_local bool t_graphs = false;
 thread_local long long t_graph_launches = 0;
@@ -48,6 +49,7 @@ cbct_ctx device_context() {
 void *current_stream() { return t_stream; }
 void set_default_storage(int dtype) { t_storage = dtype == CBCT_BF16 ? CBCT_BF16 : CBCT_F32; }
 int default_storage() { return t_storage; }
+void set_default_packed(bool on) { t_packed = on; }
 void set_default_autotune(bool on) { t_autotune = on; }
 bool default_autotune() { return t_autotune; }
 void set_default_graphs(bool on) { t_graphs = on; }
@@ -68,6 +70,7 @@ cbct_ctx acquire_context() {
     cbct_ctx c = free_list.back();
     free_list.pop_back();
     check(cbct_ctx_reset(c), c);
+    check(cbct_fp_packed(c, t_packed), c);
     return c;
   }
   cbct_ctx owner = device_context();
@@ -80,6 +83,7 @@ cbct_ctx acquire_context() {
     throw std::runtime_error(msg);
   }
   t_pool_owned[c] = dev;
+  check(cbct_fp_packed(c, t_packed), c);
   return c;
 }
 

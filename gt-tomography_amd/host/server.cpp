@@ -40,6 +40,7 @@
 #include "gtt/operators.h"
 #include "gtt/solvers.h"
 #include "gtt_c.h"
+#include "../csrc/fp_cells.h"
 #include "scan.h"
 
 using namespace gtt;
@@ -52,6 +53,7 @@ struct Job {
   long long id = 0;
   gtt_request req{};
   size_t footprint = 0;
+  bool packed = true;      // the projector's packed copy is part of it
   Clock::time_point t_submit, t_start, t_end;
   bool done = false;
   int status = 0;
@@ -76,40 +78,54 @@ double ms(Clock::time_point a, Clock::time_point b) {
 //  FDK: the image and the padded volume copy (2.3 volumes); the projections,
 //    the filtered projections, A f, the filter staging and the padded copy of
 //    all views (up to 4x as quad texels): 8 sinograms.
-//  Both: where rays leave through the volume's top or bottom, the forward
-//    projector's packed copy (4 padded volumes).
-size_t footprint_bytes(const gtt_request &r) {
+//  Both: the forward projector's packed copy where a projection (FDK: of all
+//    views; OS-SART: of a subset, taken as its worst view's times their number)
+//    builds one.  That is `packed`, and a request runs without it where only
+//    that fits the budget.
+size_t footprint_bytes(const gtt_request &r, size_t *packed) {
   const size_t nvox = (size_t)r.geom.nx * r.geom.ny * r.geom.nz;
   const size_t nproj = (size_t)(r.geom.nu + 3) * (r.geom.nv + 3) * (size_t)r.nviews;
   const size_t slack = size_t(64) << 20;
   // the LDS-staged backprojector's rectangle table: 8 bytes per 16 x 16 x 8
   // (or x 16) voxel block and view of one backprojection call
   const size_t blocks = (size_t)((r.geom.nx + 15) / 16) * ((r.geom.ny + 15) / 16) * ((r.geom.nz + 7) / 8);
-  double vtop = 0.5 * r.geom.fov_v;   // largest detector height, offsets included
-  if (r.offsets)
-    for (int k = 0; k < r.nviews; ++k)
-      vtop = std::max(vtop, 0.5 * r.geom.fov_v + std::fabs((double)r.offsets[2 * k + 1]));
-  const double R = 0.5 * std::hypot((double)r.geom.lx, (double)r.geom.ly);
-  const bool clipped = vtop * ((double)r.geom.sad + R) > 0.5 * r.geom.lz * r.geom.sdd;
-  const size_t packed = clipped ? 4 * (nvox * 52 / 10) : 0;
-  if (r.kind == GTT_REQ_FDK)
-    return 4 * (nvox * 23 / 10 + 8 * nproj) + 8 * blocks * (size_t)r.nviews + packed + slack;
   const size_t S = r.subsets > 0 ? (size_t)r.subsets : 1;
+  double rows = 0.0, worst = 0.0;   // with clipped rays
+  for (int k = 0; k < r.nviews; ++k) {
+    const double n = fp_clipped_rows(&r.geom, r.offsets ? (double)r.offsets[2 * k + 1] : 0.0);
+    rows += n;
+    worst = std::max(worst, n);
+  }
+  float spp = 1.5f;
+  if (r.kind != GTT_REQ_FDK) rows = worst * (double)(((size_t)std::max(r.nviews, 0) + S - 1) / S);
+  else if (r.samples_per_pixel > 0) spp = r.samples_per_pixel;
+  // (samples per ray beyond the projector's range are refused there)
+  const float n = std::min(spp * (float)r.geom.nx, 1e6f);
+  *packed = n >= 1.0f ? fp_cells_bytes(&r.geom, rows, (int)n, r.storage == CBCT_BF16 ? 2 : 4) : 0;
+  if (r.kind == GTT_REQ_FDK)
+    return 4 * (nvox * 23 / 10 + 8 * nproj) + 8 * blocks * (size_t)r.nviews + *packed + slack;
   return 4 * (nvox * (10 * S + 33) / 10 + 4 * nproj + 4 * ((nproj + S - 1) / S)) +
-         8 * blocks * (((size_t)r.nviews + S - 1) / S) + packed + slack;
+         8 * blocks * (((size_t)r.nviews + S - 1) / S) + *packed + slack;
 }
 
-// The request's storage type is the lane's default while its operators are
-// built (they keep it); restored afterwards.
+// The request's storage type, and whether it may hold the packed copy, are the
+// lane's defaults while its operators are built (they keep them); restored
+// afterwards.
 struct StorageScope {
   int saved;
-  explicit StorageScope(int dtype) : saved(default_storage()) { set_default_storage(dtype); }
-  ~StorageScope() { set_default_storage(saved); }
+  StorageScope(int dtype, bool packed) : saved(default_storage()) {
+    set_default_storage(dtype);
+    set_default_packed(packed);
+  }
+  ~StorageScope() {
+    set_default_storage(saved);
+    set_default_packed(true);
+  }
 };
 
 void run_request(Job &j) {
   const gtt_request &r = j.req;
-  StorageScope storage(r.storage == CBCT_BF16 ? CBCT_BF16 : CBCT_F32);
+  StorageScope storage(r.storage == CBCT_BF16 ? CBCT_BF16 : CBCT_F32, j.packed);
   // the caller's projections are only read (uploaded once), never copied
   Scan s = make_scan(&r.geom, r.angles_deg, r.offsets, r.nviews, nullptr, nullptr, 0, r.projections, true);
   if (r.kind == GTT_REQ_FDK) {
@@ -192,8 +208,9 @@ struct gtt_server_s {
         queue.pop_front();
         // the memory this lane keeps becomes part of the request's own; more
         // than the request's footprint is freed first, so that the request
-        // holds no more than its footprint says
-        trim_first = my_kept > j->footprint;
+        // holds no more than its footprint says (nor another's packed copy, where
+        // it may have none of its own)
+        trim_first = my_kept > j->footprint || (my_kept && !j->packed);
         kept -= my_kept;
         my_kept = 0;
         in_use += j->footprint;
@@ -276,7 +293,10 @@ int gtt_server_destroy(gtt_server s) {
 
 const char *gtt_server_last_error(gtt_server s) { return s ? s->err.c_str() : "null server"; }
 
-size_t gtt_request_footprint(const gtt_request *req) { return req ? footprint_bytes(*req) : 0; }
+size_t gtt_request_footprint(const gtt_request *req) {
+  size_t packed = 0;
+  return req ? footprint_bytes(*req, &packed) : 0;
+}
 
 int gtt_server_set_graphs(gtt_server s, int on) {
   if (!s) return -1;
@@ -315,7 +335,12 @@ int gtt_server_submit(gtt_server s, const gtt_request *req, long long *id) {
   j->req = *req;
   j->autotune = s->autotune;
   j->graphs = s->graphs;
-  j->footprint = footprint_bytes(*req);
+  size_t packed = 0;
+  j->footprint = footprint_bytes(*req, &packed);
+  if (j->footprint > s->budget && j->footprint - packed <= s->budget) {
+    j->footprint -= packed;
+    j->packed = false;
+  }
   if (j->footprint > s->budget) {
     s->err = "gtt_server_submit: request needs " + std::to_string(j->footprint) +
              " bytes of device memory, more than the budget of " + std::to_string(s->budget);

@@ -85,8 +85,8 @@ int cbct_ctx_trim(cbct_ctx ctx);
  * padded sinogram copy between them instead of one each.  No reference
  * counterpart (the reference allocates these per call). */
 int cbct_ctx_share_workspace(cbct_ctx ctx, cbct_ctx owner);
-/* Settings back to their defaults (engines, tile, view group, z-depth,
- * storage type, profiling); the view table, filter and scratch are kept.
+/* Settings back to their defaults (engines, tile, view group, packed
+ * copy, z-depth, storage type, profiling); the view table, filter and scratch are kept.
  * For callers that reuse contexts.  No reference counterpart. */
 int cbct_ctx_reset(cbct_ctx ctx);
 
@@ -179,6 +179,13 @@ int cbct_fp_tile(cbct_ctx ctx, int max_rows_per_lane);
  * cbct_fp_autotune also tries 1, 3, 6 and 8.  Results do not depend on it.
  * No reference counterpart. */
 int cbct_fp_view_group(cbct_ctx ctx, int views);
+
+/* Whether cbct_fp may hold a second, packed copy of the volume (four times the
+ * working copy, below 4 GB) in the workspace where many rays leave through the
+ * volume's top or bottom (default 1).  A faster call that needs more memory;
+ * results do not depend on it, and where the memory cannot be had the call does
+ * without.  No reference counterpart. */
+int cbct_fp_packed(cbct_ctx ctx, int on);
 
 /* Backprojector engine: 2 = default: LDS-staged kernels (per view, each
  * block's detector rectangle is copied into LDS by direct global-to-LDS

@@ -45,6 +45,9 @@ void release_context(cbct_ctx ctx);
 // projection operators the calling thread creates from now on (default FP32).
 void set_default_storage(int dtype);
 int default_storage();
+// Whether contexts that the calling thread acquires from now on may hold the
+// forward projector's packed volume copy (cbct_fp_packed; default on).
+void set_default_packed(bool on);
 // Whether reconstructions the calling thread starts tune the forward
 // projector for their geometry first (cbct_fp_autotune; default off).
 void set_default_autotune(bool on);

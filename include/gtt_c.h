@@ -207,7 +207,9 @@ int gtt_read_real(const char *path, float *data, size_t n);
  * gtt_server_wait() returns for it.  Admission: the head of the FIFO starts
  * once a lane is free and the estimated device footprints of the running
  * requests plus its own (gtt_request_footprint) fit the budget given at
- * creation (0: three quarters of the free device memory).
+ * creation (0: three quarters of the free device memory).  A request that
+ * fits the budget only without the projector's packed volume copy
+ * (cbct_fp_packed) runs without it.
  */
 enum { GTT_REQ_FDK = 0, GTT_REQ_OS_SART = 1 };
 

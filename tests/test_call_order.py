@@ -140,3 +140,69 @@ assert fp(h, geom(80, 80, 20, 48, 48), 30, S1) == 0 and count("free") == 0 and c
 assert L.cbct_workspace_bytes(h) == held + 4 * 83 * 83 * 32 * 4
 assert L.cbct_ctx_trim(h) == 0 and L.cbct_workspace_bytes(h) == 0
 """)
+
+
+SERVED = """
+from gtt import serving as S
+def request(kind, n, nz, nu, nv, views, offset=0.0, **more):
+    g = geom(n, n, nz, nu, nv)
+    off = np.tile(np.array([[0.0, offset]], np.float32), (views, 1))
+    return S.Request(kind=kind, geom=g, angles=angles_full(views), offsets=off, subsets=5, iterations=1,
+                     projections=np.zeros(g.proj_shape(views), np.float32), **more)
+def base(r):     # without the packed copy
+    g, v = r.geom, len(r.angles)
+    nvox, nproj = g.nx * g.ny * g.nz, (g.nu + 3) * (g.nv + 3) * v
+    blocks = -(-g.nx // 16) * -(-g.ny // 16) * -(-g.nz // 8)
+    if r.kind == S.REQ_FDK:
+        return 4 * (nvox * 23 // 10 + 8 * nproj) + 8 * blocks * v + (64 << 20)
+    return 4 * (nvox * 83 // 10 + 4 * nproj + 4 * -(-nproj // 5)) + 8 * blocks * -(-v // 5) + (64 << 20)
+def cells(r):
+    g = r.geom
+    return 4 * (g.nx + 3) * (g.ny + 3) * ((g.nz + 18) // 16 * 16) * (2 if r.storage == "bf16" else 4)
+def serve(r, budget):
+    sim.hip_log_clear()
+    with S.Server(lanes=1, hbm_budget_bytes=budget) as srv:
+        srv.wait(srv.submit(r))
+    return sum("k_fp_clip" in l for l in log())
+"""
+
+
+def test_footprint_counts_the_packed_copy_where_it_is_built(run):
+    """A request is charged for the projector's packed copy when a projection of it
+    builds one: not for a few clipped rays, not above 4 GB, by storage type."""
+    run(SERVED + """
+for kind in (S.REQ_FDK, S.REQ_OS_SART):
+    for storage in ("f32", "bf16"):
+        few = request(kind, 96, 96, 48, 36, 10, 12.0, storage=storage)      # some rays clipped
+        many = request(kind, 64, 16, 96, 96, 40, storage=storage)
+        assert few.footprint() == base(few), (kind, storage)
+        assert many.footprint() == base(many) + cells(many), (kind, storage)
+        assert serve(few, 1 << 32) == 0 and serve(many, 1 << 32) > 0
+    tall = request(kind, 900, 340, 2, 2000, 40)
+    assert cells(tall) >= 1 << 32 and tall.footprint() == base(tall)
+""")
+
+
+def test_admission_does_not_depend_on_the_packed_copy(run):
+    """A request that fits the budget without the packed copy is served without it."""
+    run(SERVED + """
+for kind in (S.REQ_FDK, S.REQ_OS_SART):
+    r = request(kind, 64, 16, 96, 96, 40)
+    assert serve(r, r.footprint()) > 0
+    assert serve(r, r.footprint() - 1) == 0 and count("launch")
+    assert serve(r, base(r)) == 0 and count("launch")
+    with S.Server(lanes=1, hbm_budget_bytes=base(r) - 1) as srv:
+        try:
+            srv.submit(r)
+            assert False
+        except RuntimeError as e:
+            assert "budget" in str(e)
+    # the next request of the lane has it again
+    with S.Server(lanes=1, hbm_budget_bytes=r.footprint() - 1) as srv:
+        srv.wait(srv.submit(r))
+        sim.hip_log_clear()
+        small = request(kind, 48, 8, 96, 96, 20)
+        assert small.footprint() < r.footprint() and small.footprint() > base(small)
+        srv.wait(srv.submit(small))
+        assert sum("k_fp_clip" in l for l in log()) > 0
+""")
