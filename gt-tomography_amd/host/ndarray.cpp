@@ -290,7 +290,8 @@ void copy_d2d(void *dst, const void *src, size_t bytes) {
 // alone), 16 MB 0.68 -> 0.57, 8 MB 0.34 -> 0.37.  Back, into fresh memory: 35 MB
 // 3.66 -> 1.45 ms, 8 MB 0.48 -> 0.36, 4 MB 0.24 -> 0.22.  So from 16 MB on and from
 // 4 MB on; smaller copies, and those whose host side is pinned already, keep
-// the runtime's path, and so does everything if no pinned memory can be had.
+// the runtime's path, and so does everything if no pinned memory can be had, or
+// on hipStreamPerThread, which names another queue in each of the threads.
 namespace {
 constexpr size_t COPY_SLOT = size_t(4) << 20, COPY_MIN_H2D = size_t(16) << 20,
                  COPY_MIN_D2H = size_t(4) << 20;
@@ -374,7 +375,9 @@ bool pageable(const void *host) {
 // for the stream, also after an error, before the slots are given back.
 bool copy_through_slots(char *dev, char *host, size_t bytes, bool to_device) {
   int d = 0;
-  if (bytes < (to_device ? COPY_MIN_H2D : COPY_MIN_D2H) || hipGetDevice(&d) != hipSuccess || !pageable(host)) return false;
+  if (bytes < (to_device ? COPY_MIN_H2D : COPY_MIN_D2H) || t_stream == hipStreamPerThread ||
+      hipGetDevice(&d) != hipSuccess || !pageable(host))
+    return false;
   CopySlots *c = take_slots(d);
   if (!c) return false;
   const hipStream_t s = t_stream;

@@ -206,3 +206,37 @@ for kind in (S.REQ_FDK, S.REQ_OS_SART):
         srv.wait(srv.submit(small))
         assert sum("k_fp_clip" in l for l in log()) > 0
 """)
+
+
+COPIES = """
+import os, threading
+from gtt import operators as ops
+G = ops.load()
+h2d, d2h, stream = G._ZN3gtt8copy_h2dEPvPKvm, G._ZN3gtt8copy_d2hEPvPKvm, G._ZN3gtt18set_current_streamEPv
+trim, release = G._ZN3gtt18trim_thread_memoryEv, G._ZN3gtt24release_thread_resourcesEv
+for f in (h2d, d2h):
+    f.argtypes, f.restype = [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_size_t], None
+for f in (stream, trim, release):
+    f.argtypes, f.restype = [ctypes.c_void_p] if f is stream else [], None
+MB = 1 << 20
+def copies():      # (stream, thread) of each
+    return [(int(l.split()[1], 0) if l.split()[1] != "(nil)" else 0, int(l.split()[4])) for l in log() if l.startswith("copy")]
+"""
+
+
+def test_host_copies_on_the_threads_own_default_stream(run):
+    """hipStreamPerThread is another queue in every thread: the calling thread alone
+    queues the copies."""
+    run(COPIES + """
+a, b = np.arange(32 * MB, dtype=np.uint8), np.zeros(32 * MB, np.uint8)
+me = threading.get_native_id()
+for s, alone in ((S1, False), (2, True)):
+    stream(s)
+    for f in (h2d, d2h):
+        sim.hip_log_clear()
+        b[:] = 0
+        f(b.ctypes.data, a.ctypes.data, b.size)
+        assert np.array_equal(a, b)
+        assert {c[0] for c in copies()} == {s}
+        assert ({c[1] for c in copies()} == {me}) or not alone
+""")
