@@ -378,9 +378,12 @@ bool copy_through_slots(char *dev, char *host, size_t bytes, bool to_device) {
   if (bytes < (to_device ? COPY_MIN_H2D : COPY_MIN_D2H) || t_stream == hipStreamPerThread ||
       hipGetDevice(&d) != hipSuccess || !pageable(host))
     return false;
+  const hipStream_t s = t_stream;
+  // back to the host: earlier work is waited for here, once, and not by every
+  // helper on its first event, with slots taken
+  if (!to_device) hip_check(hipStreamSynchronize(s), "hipStreamSynchronize");
   CopySlots *c = take_slots(d);
   if (!c) return false;
-  const hipStream_t s = t_stream;
   // an eighth of the copy, but 1 MB to a slot: each chunk costs about 14 us more
   // than its time on the bus, and a last copy on the host is not hidden
   const size_t eighth = (bytes / (2 * COPY_THREADS) + 4095) / 4096 * 4096;

@@ -240,3 +240,17 @@ for s, alone in ((S1, False), (2, True)):
         assert {c[0] for c in copies()} == {s}
         assert ({c[1] for c in copies()} == {me}) or not alone
 """)
+
+
+def test_copies_back_wait_once(run):
+    """A copy back to the host waits for the stream's earlier work on the calling thread,
+    before any helper does: no helper waits for more than its own chunks."""
+    run(COPIES + """
+a, b = np.arange(32 * MB, dtype=np.uint8), np.zeros(32 * MB, np.uint8)
+stream(S1)
+sim.hip_log_clear()
+d2h(b.ctypes.data, a.ctypes.data, b.size)
+assert np.array_equal(a, b)
+lines = [l.split() for l in log() if l.split()[0] in ("copy", "sync_stream", "sync_event")]
+assert lines[0] == ["sync_stream", hex(S1), str(threading.get_native_id())], lines[0]
+""")
