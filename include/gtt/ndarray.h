@@ -72,7 +72,8 @@ void trim_device_cache();
 // blocks and the scratch of its contexts on the current device.
 size_t retained_device_bytes();
 // Frees both (after the thread's last calls that used them have finished).  Also
-// frees the pinned slots that host copies of any thread have left idle.
+// frees the pinned slots of host copies beyond one set for each other thread
+// that copies.
 void trim_thread_memory();
 // Executable HIP graph of the device work a function queues on the calling
 // thread's current stream (which must not be the default stream: it cannot

@@ -254,3 +254,41 @@ assert np.array_equal(a, b)
 lines = [l.split() for l in log() if l.split()[0] in ("copy", "sync_stream", "sync_event")]
 assert lines[0] == ["sync_stream", hex(S1), str(threading.get_native_id())], lines[0]
 """)
+
+
+def test_pinned_slots_are_kept_for_copies_at_once(run):
+    """Slots are pinned for the copies that run at once, up to eight, and kept while the
+    threads that copy are there; a thread's trim or end frees no others'."""
+    run(COPIES + """
+def work(n, gate, ok, done):
+    a = np.arange(20 * MB, dtype=np.uint8)
+    b = np.zeros_like(a)
+    stream(S1)
+    for r in range(6):
+        gate.wait()
+        d2h(b.ctypes.data, a.ctypes.data, b.size)
+    ok.append(np.array_equal(a, b))
+    gate.wait()      # the log is looked at
+    gate.wait()
+    release()
+    done.wait()
+for n in (1, 5, 12):
+    sim.hip_log_clear()
+    gate, done, ok = threading.Barrier(n + 1), threading.Barrier(n + 1), []
+    ts = [threading.Thread(target=work, args=(n, gate, ok, done), daemon=True) for _ in range(n)]
+    for t in ts:
+        t.start()
+    for r in range(6):
+        gate.wait()
+    gate.wait()
+    assert len(ok) == n and all(ok)
+    made = count("host_malloc")
+    assert made <= min(n, 8) and count("host_free") == 0, (n, made, count("host_free"))
+    trim()           # this thread copies nothing
+    assert count("host_free") == 0
+    gate.wait()
+    done.wait()
+    assert count("host_free") == made, (made, count("host_free"))
+    for t in ts:
+        t.join()
+""")
