@@ -7,12 +7,12 @@
 #include <algorithm>
 #include <atomic>
 #include <cstring>
+#include <exception>
 #include <map>
 #include <mutex>
 #include <new>
 #include <set>
 #include <string>
-#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -451,7 +451,7 @@ bool copy_through_slots(char *dev, char *host, size_t bytes, bool to_device) {
   std::thread helpers[COPY_THREADS];
   try {
     for (int t = 1; t < COPY_THREADS; ++t) helpers[t] = std::thread(work, t);
-  } catch (const std::system_error &) {   // no more threads: those there are share the chunks
+  } catch (const std::exception &) {   // no more threads, or no memory for one: those there are share the chunks
   }
   work(0);
   for (auto &h : helpers)
