@@ -1316,11 +1316,15 @@ FPChoice select_variant(cbct_ctx ctx, const cbct_geom *g, const FPParams &P, int
   const int per_step = esz == 2 ? 2 : 1;
   if (ctx->fp_engine == 2) return {3 - per_step, rpl};
   if (ctx->fp_engine >= 3) return {3, rpl, ctx->fp_engine == 3 ? 4 : 6};
+  FPChoice tuned{0, 0};
   {
     std::lock_guard<std::mutex> lk(g_tune_mu);
     auto it = g_tuned.find(tune_key(g, spp, esz));
-    if (it != g_tuned.end()) return it->second.choice;
+    if (it != g_tuned.end()) tuned = it->second.choice;
   }
+  // the key holds no detector offsets: a tuned tile's window is the call's own
+  if (tuned.variant == 3) tuned.zc = window_zc(ctx, g, P.nv, tuned.rpl, view0, nviews);
+  if (tuned.variant && tuned.zc <= FP_ZC_MAX) return tuned;
   return default_variant(ctx, g, P, view0, nviews, esz, per_step);
 }
 

@@ -292,3 +292,38 @@ for n in (1, 5, 12):
     for t in ts:
         t.join()
 """)
+
+
+def test_tuned_window_follows_the_offsets(run):
+    """A tuned forward projector takes the z window that the views of the call need, not
+    the one of the views it was tuned with; where no window of its tile holds them it
+    takes what an untuned one takes."""
+    run("""
+import re
+nviews, g = 5, geom(12, 12, 500, 14, 70, fov=(24.0, 90.0))
+h = context()
+def offsets(v):
+    views(h, angles_full(nviews), np.stack([np.zeros(nviews), np.linspace(-v, v, nviews)], 1))
+def kernel():     # (name, template arguments: rows and z per lane, steps in flight)
+    sim.hip_log_clear()
+    assert fp(h, g, nviews, S1) == 0
+    m, = [m for m in (re.search("k_fp_colc?IfLi(.*?)EEEv", l) for l in log()) if m]
+    return m.group(0), [int(x) for x in re.findall("[0-9]+", m.group(0).split("If", 1)[1])]
+spans = (0.0, 20.0, 60.0, 150.0, 330.0, 0.0)
+plain = []
+for v in spans:
+    offsets(v)
+    plain.append((L.cbct_fp_kernel(h, ctypes.byref(g), 0, nviews, 0, 1.5), kernel()))
+zc = [k[1][1][1] for k in plain[:4]]
+assert zc == sorted(zc) and zc[0] < zc[-1] and plain[4][0] == b"k_fp_col", plain
+for tune in range(4):
+    L.cbct_fp_autotune_clear()
+    offsets(spans[tune])
+    best = ctypes.c_double()
+    assert L.cbct_fp_autotune(h, ctypes.byref(g), 0, nviews, 0, 1.5, 0, S1, ctypes.byref(best)) == 0
+    for v, p in zip(spans, plain):
+        offsets(v)
+        assert L.cbct_fp_kernel(h, ctypes.byref(g), 0, nviews, 0, 1.5) == p[0], (tune, v)
+        k = kernel()
+        assert k[0] == p[1][0] or k[1][0] != p[1][1][0], (tune, v, k, p)
+""")
