@@ -7,8 +7,9 @@
 // evaluating the projected gradient once per voxel.  The dual's p(v-ey) and
 // p(v-ez) are the thread's own from the row before and the slice before,
 // p(v-ex) is the neighbouring lane's.  HBM traffic per voxel is 3 floats (read
-// x, read + write out).  The arithmetic per gradient is the reference's, in
-// the same order, so the fused result equals the two-kernel result.
+// x, read + write out).  The arithmetic is the reference's, in the same order,
+// but for the divisions by the norm (tv_grad), which may differ from plain ones in
+// the last bit.
 #include "cbct_internal.h"
 
 namespace {
