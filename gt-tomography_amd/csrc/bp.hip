@@ -783,11 +783,20 @@ int run_bp(cbct_ctx ctx, const cbct_geom *g, BPParams P, dim3 grid, int kz, int 
     const int vec = g->nu % 4 == 0 && reinterpret_cast<uintptr_t>(proj) % (4 * sizeof(TI)) == 0;
     const ViewF *vf = ctx->d_views_f + view0;
     const dim3 pad = pad_grid(P.pnu2 / 4, nviews);
-    const size_t rect_blocks = (nblocks * nviews + 255) / 256, prep = rect_blocks + (size_t)pad.x * pad.y * pad.z;
+    const size_t rect_blocks = (nblocks * nviews + 255) / 256, pad_blocks = (size_t)pad.x * pad.y * pad.z;
     const auto k_prep = kz == 8 ? k_bpp_prep<TI, PAIRS, 8> : k_bpp_prep<TI, PAIRS, KZ>;
-    hipLaunchKernelGGL(k_prep, dim3((unsigned)prep), dim3(256), 0, s, P, vf, rects, grid.x, grid.y,
-                       (unsigned)nblocks, (unsigned)rect_blocks, proj, cp, g->nu, g->nv, vec,
-                       make_uint3(pad.x, pad.y, pad.z));
+    auto prep = [&](size_t rect, size_t padding) {
+      hipLaunchKernelGGL(k_prep, dim3((unsigned)(rect + padding)), dim3(256), 0, s, P, vf, rects, grid.x, grid.y,
+                         (unsigned)nblocks, (unsigned)rect, proj, cp, g->nu, g->nv, vec,
+                         make_uint3(pad.x, pad.y, pad.z));
+    };
+    if ((rect_blocks + pad_blocks) * 256 < 1ull << 32) {
+      prep(rect_blocks, pad_blocks);
+    } else {   // more than a launch holds
+      prep(rect_blocks, 0);
+      CBCT_LAUNCH_CHECK(ctx, "k_bpp_prep");
+      prep(0, pad_blocks);
+    }
     CBCT_LAUNCH_CHECK(ctx, "k_bpp_prep");
     cbct_prof_mark(ctx, PROF_BP, 0, s);
     if (kz == 8)

@@ -125,7 +125,12 @@ int hipGetDevice(int *d) { *d = 0; return SUCCESS; }
 int hipSetDevice(int d) { return d ? INVALID : SUCCESS; }
 int hipDeviceGetAttribute(int *v, int a, int d) { *v = 256; return SUCCESS; }
 int hipOccupancyMaxActiveBlocksPerMultiprocessor(int *n, const void *f, int b, size_t s) { *n = 2; return SUCCESS; }
-int hipGetLastError(void) { return SUCCESS; }
+static __thread int last_error;
+int hipGetLastError(void) {
+  int e = last_error;
+  last_error = SUCCESS;
+  return e;
+}
 const char *hipGetErrorString(int e) { return e == OUT_OF_MEMORY ? "out of memory" : e == CAPTURE ? "capturing" : "error"; }
 static char symbol[64 << 20];
 int hipGetSymbolAddress(void **p, const void *s) { *p = symbol; return SUCCESS; }
@@ -157,7 +162,8 @@ int hipLaunchKernel(const void *f, dim3 g, dim3 b, void **args, size_t m, void *
   for (int i = 0; i < kernels; ++i)
     if (kernel[i].f == f) name = kernel[i].name;
   say("launch %p %u %u %u %u %.180s", s, g.x, g.y, g.z, b.x * b.y * b.z, name);
-  return (uint64_t)g.x * b.x >> 32 ? INVALID : SUCCESS;
+  if ((uint64_t)g.x * b.x >> 32) last_error = INVALID;
+  return last_error;
 }
 
 /* ---- graphs: not simulated */

@@ -327,3 +327,20 @@ for tune in range(4):
         k = kernel()
         assert k[0] == p[1][0] or k[1][0] != p[1][1][0], (tune, v, k, p)
 """)
+
+
+def test_backprojection_of_many_block_views(run):
+    """A launch holds less than 2^32 work-items: block-views just below that and the
+    padded copy's blocks are more together, but not each alone."""
+    run("""
+n = 65535
+h = context(angles_full(n))
+for g in (geom(512, 512, 1008, 1, 1), geom(512, 512, 1024, 1, 1)):
+    sim.hip_log_clear()
+    assert bp(h, g, n, S1) == 0, L.cbct_last_error(h)
+    prep = [l.split() for l in log() if "k_bpp_prep" in l]
+    blocks = 32 * 32 * (g.nz // 16)
+    assert len(prep) == (1 if g.nz < 1024 else 2)
+    assert sum(int(w[2]) for w in prep) == blocks * n // 256 + 16 * 1024 and "k_bpp" in log()[-2]
+    assert L.cbct_ctx_trim(h) == 0
+""")
