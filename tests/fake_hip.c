@@ -10,6 +10,7 @@
 #include <stdlib.h>
 #include <string.h>
 #include <unistd.h>
+#include <sys/mman.h>
 #include <sys/syscall.h>
 
 enum { SUCCESS = 0, OUT_OF_MEMORY = 2, INVALID = 1, CAPTURE = 900 };
@@ -45,7 +46,11 @@ size_t hip_live;
 
 static int take(void **p, size_t n, int host) {
   pthread_mutex_lock(&mu);
-  int ok = (host || hip_live + n <= hip_limit) && blocks < 4096 && (*p = malloc(n ? n : 1));
+  int ok = (host || hip_live + n <= hip_limit) && blocks < 4096;
+  if (ok) {   /* pages are there when they are used, if ever */
+    *p = mmap(0, n ? n : 1, PROT_READ | PROT_WRITE, MAP_PRIVATE | MAP_ANONYMOUS | MAP_NORESERVE, -1, 0);
+    ok = *p != MAP_FAILED;
+  }
   if (ok) {
     block[blocks].p = *p;
     block[blocks].n = n;
@@ -62,11 +67,11 @@ static void drop(void *p) {
   for (int i = 0; i < blocks; ++i)
     if (block[i].p == p) {
       if (!block[i].host) hip_live -= block[i].n;
+      munmap(p, block[i].n ? block[i].n : 1);
       block[i] = block[--blocks];
       break;
     }
   pthread_mutex_unlock(&mu);
-  free(p);
 }
 
 static void *capturing[16];
