@@ -27,9 +27,10 @@
 //  instruction) into LDS, and every ray then does one z-lerp from LDS.  The
 //  arithmetic order (x-lerps, y-lerp, z-lerp) and sample coordinates are those
 //  of engine 0, so both engines produce bitwise-identical projections.  Rays
-//  clipped by the z slab run the per-ray loop.  Blocks are remapped so each
-//  XCD walks a contiguous run of columns (neighbouring columns share z-lines
-//  in that XCD's L2).
+//  clipped by the z slab are taken 8 samples of 8 rays at a time (fp_gather),
+//  where they are many by a kernel of their own (k_fp_clip).  Blocks are remapped
+//  so each XCD walks a contiguous run of columns (neighbouring columns share
+//  z-lines in that XCD's L2).
 //
 // Engine 0: one thread per ray, 16x16 detector tiles, x-fastest padded
 // volume, 8 gathers per sample.  Also the basis of the exact transpose.
@@ -226,11 +227,6 @@ __global__ void __launch_bounds__(256) k_fp_ray_transpose(FPParams P, const View
 }
 
 // ------------------------------------------------------------------ engine 1
-__device__ __forceinline__ float wave_min(float v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v = fminf(v, __shfl_xor(v, o, 64));
-  return v;
-}
 __device__ __forceinline__ int wave_min_i(int v) {
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) v = min(v, __shfl_xor(v, o, 64));
@@ -558,7 +554,7 @@ __device__ __forceinline__ void col_block(const FPParams &P, unsigned W, unsigne
 //   SSTEP = false, ZP = 1: per-step setup on the vector unit, one z per lane
 //     and load (FP32 storage: measured fastest there).
 //   SSTEP = true, ZP = 2: integer step setup in scalar registers, no per-ray
-//     z clamp (a column-level range check instead), two consecutive z per
+//     z clamp (shared rays stay inside the volume's z), two consecutive z per
 //     lane and load (BF16 storage: one dword per lane instead of two 16-bit
 //     loads, 1.5x faster there).
 //   ZC > 0 (with SSTEP, ZP = 2): the z window of the whole ray (all its steps,
@@ -726,7 +722,7 @@ __device__ __forceinline__ void fp_col_body(const FPParams &P, const ViewD *__re
           auto rays = [&](const float fm) __attribute__((always_inline)) {
 #pragma unroll
               for (int r = 0; r < RPL; ++r) {
-                const float tz = fmaf(fm, qz[r], pz[r]);  // in [0, nz+1]: checked above
+                const float tz = fmaf(fm, qz[r], pz[r]);  // in [0, nz+1]: as above
                 const int iz = (int)tz;
                 const float az = __builtin_amdgcn_fractf(tz);
                 const float a = zb[iz], b = zb[iz + 1];
@@ -826,7 +822,7 @@ __device__ __forceinline__ void fp_col_body(const FPParams &P, const ViewD *__re
       const float *zb = zl - zb0;
 #pragma unroll
       for (int r = 0; r < RPL; ++r) {
-        const float tz = fmaf(fm, qz[r], pz[r]);  // in [0, nz+1]: checked above
+        const float tz = fmaf(fm, qz[r], pz[r]);  // in [0, nz+1]: as above
         const int iz = (int)tz;
         const float az = __builtin_amdgcn_fractf(tz);
         const float a = zb[iz], b = zb[iz + 1];
