@@ -647,9 +647,9 @@ struct FftRadix {
   static constexpr int R = N / NS >= P ? P : N / NS;
 };
 
-// twiddles a butterfly keeps: all R - 1 (the kernel is bound by vector
-// instruction issue and holds two waves per SIMD, so registers are cheaper
-// than forming twiddles as products in every pass)
+// twiddles a butterfly keeps: all R - 1 (the kernel holds two waves per SIMD, so
+// registers are cheaper than forming twiddles as products in every pass: 1.54-1.58
+// -> 1.47-1.52 ms at 552,960 rows of 1024)
 template <int R>
 struct FftKeep {
   static constexpr int value = R - 1;
