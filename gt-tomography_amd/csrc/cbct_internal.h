@@ -80,6 +80,7 @@ struct cbct_ctx_s {
   bool done_recorded = false;
   CallEvent noalloc_done;
   bool noalloc_recorded = false;
+  bool captured = false;         // a call was captured into a graph: no event marks its replays
   // filter state
   int filter_nu = 0;
   int filter_engine = 2;

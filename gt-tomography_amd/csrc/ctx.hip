@@ -141,6 +141,7 @@ bool cbct_capturing(hipStream_t s) {
 
 CallScope::CallScope(cbct_ctx c, hipStream_t st) : ctx(c), s(st), capturing(cbct_capturing(st)) {
   Workspace &w = *ctx->ws;
+  if (capturing) ctx->captured = true;
   if (!capturing && w.done && w.last != s) (void)hipStreamWaitEvent(s, w.done->e, 0);
 }
 
@@ -271,6 +272,7 @@ int cbct_ctx_reset(cbct_ctx ctx) {
   ctx->fp_force_zc = d.fp_force_zc;
   ctx->fp_force_vg = d.fp_force_vg;
   ctx->work_dtype = d.work_dtype;
+  ctx->captured = false;
   ctx->profile = false;
   for (bool &r : ctx->ev_recorded) r = false;
   ctx->err.clear();

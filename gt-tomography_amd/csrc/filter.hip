@@ -1258,9 +1258,10 @@ int cbct_filter_set(cbct_ctx ctx, int nu, const float *F) {
   std::vector<double> h = spatial_kernel(nu, F);
   std::vector<float> hm(2 * (size_t)nu - 1);
   for (int d = -(nu - 1); d <= nu - 1; ++d) hm[d + nu - 1] = (float)h[d < 0 ? -d : d];
-  // calls still reading the old tables finish first
+  // calls still reading the old tables finish first, and replays of captured ones
   rc = cbct_wait_tables(ctx);
   if (rc) return rc;
+  if (ctx->captured) CBCT_HIP_CHECK(ctx, hipDeviceSynchronize());
   // (their memory is kept where the new ones are of the same size)
   if (ctx->d_h && ctx->h64.size() != (size_t)nu) {
     (void)hipFree(ctx->d_h);

@@ -25,7 +25,8 @@
  *    when that was enqueued on another stream, so the scratch is never
  *    overwritten while a kernel still reads it.  cbct_views_set and
  *    cbct_filter_set wait (on the host) for this context's earlier calls
- *    only, not for the whole device.
+ *    only, not for the whole device (cbct_filter_set for the device where a
+ *    call on the context has been captured into a graph).
  */
 #ifndef CBCT_H
 #define CBCT_H
@@ -87,6 +88,7 @@ int cbct_ctx_trim(cbct_ctx ctx);
 int cbct_ctx_share_workspace(cbct_ctx ctx, cbct_ctx owner);
 /* Settings back to their defaults (engines, tile, view group, packed
  * copy, z-depth, storage type, profiling); the view table, filter and scratch are kept.
+ * Replays of graphs that hold the context's calls must have finished.
  * For callers that reuse contexts.  No reference counterpart. */
 int cbct_ctx_reset(cbct_ctx ctx);
 

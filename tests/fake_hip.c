@@ -114,7 +114,7 @@ int hipStreamCreate(void **s) { *s = malloc(1); return SUCCESS; }
 int hipStreamCreateWithFlags(void **s, unsigned f) { *s = malloc(1); return SUCCESS; }
 int hipStreamDestroy(void *s) { return SUCCESS; }
 int hipStreamSynchronize(void *s) { say("sync_stream %p %ld", s, (long)syscall(SYS_gettid)); return is_capturing(s) ? CAPTURE : SUCCESS; }
-int hipDeviceSynchronize(void) { say("sync_device"); return SUCCESS; }
+int hipDeviceSynchronize(void) { say("sync_device"); return captures ? CAPTURE : SUCCESS; }
 int hipStreamIsCapturing(void *s, int *st) { *st = is_capturing(s); return SUCCESS; }
 int hipStreamWaitEvent(void *s, void *e, unsigned f) { say("wait %p %p", s, e); return SUCCESS; }
 int hipEventCreateWithFlags(void **e, unsigned f) { *e = malloc(1); say("event_create %p", *e); return SUCCESS; }

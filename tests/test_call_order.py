@@ -344,3 +344,26 @@ for g in (geom(512, 512, 1008, 1, 1), geom(512, 512, 1024, 1, 1)):
     assert sum(int(w[2]) for w in prep) == blocks * n // 256 + 16 * 1024 and "k_bpp" in log()[-2]
     assert L.cbct_ctx_trim(h) == 0
 """)
+
+
+def test_filter_waits_for_replays(run):
+    """A filter is replaced in place, also where a captured call reads it: no event marks
+    a replay's end, so the device is waited for then, and only then."""
+    run("""
+g = geom(16, 16, 16, 32, 24)
+h = context(angles_full(6), filt=32)
+assert prefilter(h, g, 6, S1) == 0 and set_filter(h, 32) == 0 and count("sync_device") == 0
+assert prefilter(h, g, 6, S1) == 0
+sim.hip_capture(S1, 1)
+assert prefilter(h, g, 6, S1) == 0
+sim.hip_capture(S1, 0)
+for _ in range(2):
+    sim.hip_log_clear()
+    assert set_filter(h, 32) == 0
+    first = [l.split()[0] for l in log() if l.split()[0] in ("sync_device", "copy")]
+    assert first[0] == "sync_device", first
+    # the tables made from it on the next call come after that
+    sim.hip_log_clear()
+    assert prefilter(h, g, 6, S1) == 0 and count("sync_device") == 0
+assert L.cbct_ctx_reset(h) == 0 and set_filter(h, 32) == 0 and count("sync_device") == 0
+""")
